@@ -372,9 +372,44 @@ class BatchPlan:
         self.nops = len(host_ops)
         self.nleaves = len(host_leaves)
         self.program_shape = _program_shape(recs, self.host_ops, self.host_leaves)
+        self.stamp_groups, self.list_groups = self._split_groups()
         self._sched = None
         self._graph = None
         self.tuning = None
+
+    def _split_groups(self):
+        """(stamp groups, list groups): the FFT sizes each of whose stamps one workgroup draws in
+        one kernel (N, first, count, largest Nk, Sersic coefficients; gsmi_draw_stamps_f32) and
+        the (N, first, count, max_ny) of the fold and row kernels.  The one-kernel form takes
+        FP32 batches of a specialised program shape at N = 128 and 192, whose wrapped grid fits
+        one workgroup's LDS, while Nk < 2 N (at most one alias per axis, which is what its cell
+        passes add)."""
+        if self.precision != 'f32' or not self.program_shape:
+            return [], list(self.groups)
+        ncoef = 0
+        sel = self.host_leaves['type'] == _lib.LEAF_SERSIC
+        if sel.any():
+            if np.any(self.host_leaves['cliprows'][sel] < 0):
+                return [], list(self.groups)
+            ncoef = int(self.host_leaves['ntab'][sel].max()) - 1
+        one, two = [], []
+        lds = _lib.lib().gsmi_draw_stamps_lds
+        for N, first, count, max_ny in self.groups:
+            nk = int(self.recs['Nk'][first:first + count].max())
+            if 0 < lds(N, nk, ncoef) <= LIST_LDS_LIMIT:
+                one.append((N, first, count, nk, ncoef))
+            else:
+                two.append((N, first, count, max_ny))
+        return one, two
+
+    def _launch_stamps(self, group, s):
+        N, first, count, nk, ncoef = group
+        base = self.dev.data_ptr()
+        rc = _lib.lib().gsmi_draw_stamps_f32(
+            base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize, count, N, nk, ncoef,
+            self.program_shape, base + self._o_ops, base + self._o_leaves, base + self._o_tab,
+            base + self._o_tab32, self.out.data_ptr(), s)
+        _lib.check(rc, "batched stamps (N=%d)" % N)
 
     # -- work-list schedule ----------------------------------------------------------------------
     @staticmethod
@@ -409,12 +444,12 @@ class BatchPlan:
         sizes and the program shape to launch."""
         extra = self._fold_extra()
         try:
-            return work_lists(self.recs, self.groups, cols, rows, self._elem(), bins, chunks,
+            return work_lists(self.recs, self.list_groups, cols, rows, self._elem(), bins, chunks,
                               extra) + (self.program_shape,)
         except _lib.GalSimAMDError:
             if not extra:
                 raise
-        return work_lists(self.recs, self.groups, cols, rows, self._elem(), bins, chunks,
+        return work_lists(self.recs, self.list_groups, cols, rows, self._elem(), bins, chunks,
                           0) + (0,)
 
     def make_schedule(self, cols=None, rows=None, fold_grid=None, rows_grid=None, bins=None,
@@ -449,10 +484,13 @@ class BatchPlan:
         lib = _lib.lib()
         base = self.dev.data_ptr()
         sc = ctypes.addressof(sched[1])
+        if part in ('fold', 'all'):
+            for group in self.stamp_groups:
+                self._launch_stamps(group, s)
         args_fold = (base + self._o_stamp, self.nrec, sc, base + self._o_ops,
                      base + self._o_leaves,
                      base + self._o_tab)
-        if part in ('fold', 'all'):
+        if part in ('fold', 'all') and self.list_groups:
             if self.precision == 'f32':
                 rc = lib.gsmi_fold_list_f32(*args_fold, base + self._o_tab32,
                                             self.scratch.data_ptr(), s)
@@ -460,7 +498,7 @@ class BatchPlan:
                 rc = lib.gsmi_fold_list_f64(*args_fold, base + self._o_clip,
                                             self.scratch.data_ptr(), s)
             _lib.check(rc, "fold work list")
-        if part in ('rows', 'all'):
+        if part in ('rows', 'all') and self.list_groups:
             f = lib.gsmi_rows_list_f32 if self.precision == 'f32' else lib.gsmi_rows_list_f64
             rc = f(base + self._o_stamp, self.nrec, sc, self.scratch.data_ptr(),
                    self.out.data_ptr(), s)
@@ -491,7 +529,7 @@ class BatchPlan:
         s = torch.cuda.current_stream().cuda_stream
         cols, rows, log = {}, {}, {}
         elem = self._elem()
-        for N, first, count, _ in self.groups:
+        for N, first, count, _ in self.list_groups:
             W = N // 2               # fold columns (kx = 0 and kx = N/2 packed as one)
             best = None
             # powers of two around the default, and widths that split the W columns into
@@ -529,7 +567,7 @@ class BatchPlan:
         # this size vary by a few percent from run to run)
         combos = []
         for cells in item_cells:
-            ck = {N: max(1, cells // (cols[N] * N)) for N, _, _, _ in self.groups}
+            ck = {N: max(1, cells // (cols[N] * N)) for N, _, _, _ in self.list_groups}
             for g in grids:
                 sched = self.make_schedule(cols, rows, g, g, chunks=ck)
                 t = self._time(lambda: self._launch_list(sched, 'all', s), reps)
@@ -601,7 +639,13 @@ class BatchPlan:
             if events:
                 events('end', 0).record()
             return self.out
-        for N, first, count, max_ny in self.groups:
+        for group in self.stamp_groups:
+            if events:
+                events('fold', group[0]).record()
+            self._launch_stamps(group, s)
+            if events:
+                events('rows', group[0]).record()
+        for N, first, count, max_ny in self.list_groups:
             st = base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize
             if events:
                 events('fold', N).record()

@@ -367,6 +367,19 @@ int gsmi_rows_list_f64(const gsmi_stamp* stamps, int nstamps, const gsmi_schedul
 int gsmi_rows_list_f32(const gsmi_stamp* stamps, int nstamps, const gsmi_schedule* sched,
                        const void* scratch, float* out, void* stream);
 
+/* Draw nstamps FP32 stamps of one FFT size N (128 or 192), each by one workgroup that keeps the
+ * stamp's wrapped grid in LDS from the k-space samples to the pixels: no scratch buffer and one
+ * launch.  The same drawing as gsmi_draw_list_f32 (axis factors, status word and output offsets
+ * included).  Every stamp has N <= Nk <= max_Nk < 2 N, the shape of the nonzero
+ * gsmi_schedule.program given and a Sersic table (if the shape has one) with at most max_ncoef
+ * coefficient quadruples; a stamp that breaks this is left undrawn with GSMI_STAMP_NONFINITE set.
+ * GSMI_E_SIZE for another N or beyond the device's LDS. */
+int gsmi_draw_stamps_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int max_ncoef,
+                         int program, const gsmi_op* ops, const gsmi_leaf* leaves,
+                         const double* tables, const float* tables32, float* out, void* stream);
+/* LDS bytes of one workgroup of gsmi_draw_stamps_f32, or -1 for sizes it does not take. */
+int64_t gsmi_draw_stamps_lds(int N, int max_Nk, int max_ncoef);
+
 /* Evaluate a stamp program on a k-image with bounds (xmin..xmin+nx-1, ymin..ymin+ny-1) and
  * spacing dk, writing complex128 values row-major (SBProfile::drawK src/SBProfile.cpp:383-425
  * through the Python _drawKImage tree, gsobject.py:2464-2583 drawKImage). */
