@@ -372,44 +372,56 @@ class BatchPlan:
         self.nops = len(host_ops)
         self.nleaves = len(host_leaves)
         self.program_shape = _program_shape(recs, self.host_ops, self.host_leaves)
-        self.stamp_groups, self.list_groups = self._split_groups()
+        self.stamp_groups, self.wide_groups, self.list_groups = self._split_groups()
         self._sched = None
         self._graph = None
         self.tuning = None
 
     def _split_groups(self):
-        """(stamp groups, list groups): the FFT sizes each of whose stamps one workgroup draws in
-        one kernel (N, first, count, largest Nk, Sersic coefficients; gsmi_draw_stamps_f32) and
-        the (N, first, count, max_ny) of the fold and row kernels.  The one-kernel form takes
-        FP32 batches of a specialised program shape at N = 128 and 192, whose wrapped grid fits
-        one workgroup's LDS, while Nk < 2 N (at most one alias per axis, which is what its cell
-        passes add)."""
+        """(stamp groups, wide groups, list groups): how each FFT size is drawn.  FP32 batches of
+        a specialised program shape whose stamps have Nk < 2 N (at most one alias per axis, which
+        is what the cell passes of these kernels add) take the kernels compiled per size: one
+        workgroup per stamp at N = 128 and 192, whose wrapped grid fits its LDS
+        (gsmi_draw_stamps_f32), a column and a row kernel from 256 to 4096 (gsmi_draw_wide_f32);
+        both (N, first, count, max_ny, largest Nk, Sersic coefficients).  Everything else, as
+        (N, first, count, max_ny), takes the fold and row kernels of any shape and size."""
         if self.precision != 'f32' or not self.program_shape:
-            return [], list(self.groups)
+            return [], [], list(self.groups)
         ncoef = 0
         sel = self.host_leaves['type'] == _lib.LEAF_SERSIC
         if sel.any():
             if np.any(self.host_leaves['cliprows'][sel] < 0):
-                return [], list(self.groups)
+                return [], [], list(self.groups)
             ncoef = int(self.host_leaves['ntab'][sel].max()) - 1
-        one, two = [], []
-        lds = _lib.lib().gsmi_draw_stamps_lds
+        one, wide, rest = [], [], []
+        lib = _lib.lib()
         for N, first, count, max_ny in self.groups:
             nk = int(self.recs['Nk'][first:first + count].max())
-            if 0 < lds(N, nk, ncoef) <= LIST_LDS_LIMIT:
-                one.append((N, first, count, nk, ncoef))
+            if 0 < lib.gsmi_draw_stamps_lds(N, nk, ncoef) <= LIST_LDS_LIMIT:
+                one.append((N, first, count, max_ny, nk, ncoef))
+            elif 0 < lib.gsmi_draw_wide_lds(N, nk, ncoef) <= LIST_LDS_LIMIT:
+                wide.append((N, first, count, max_ny, nk, ncoef))
             else:
-                two.append((N, first, count, max_ny))
-        return one, two
+                rest.append((N, first, count, max_ny))
+        return one, wide, rest
 
-    def _launch_stamps(self, group, s):
-        N, first, count, nk, ncoef = group
+    def _launch_sized(self, s, mark=None):
+        """The stamp and wide groups' launches on stream ``s``; ``mark(N)``, if given, is called
+        before each size's."""
+        lib = _lib.lib()
         base = self.dev.data_ptr()
-        rc = _lib.lib().gsmi_draw_stamps_f32(
-            base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize, count, N, nk, ncoef,
-            self.program_shape, base + self._o_ops, base + self._o_leaves, base + self._o_tab,
-            base + self._o_tab32, self.out.data_ptr(), s)
-        _lib.check(rc, "batched stamps (N=%d)" % N)
+        o = (self.program_shape, base + self._o_ops, base + self._o_leaves, base + self._o_tab,
+             base + self._o_tab32)
+        for N, first, count, max_ny, nk, ncoef in self.stamp_groups + self.wide_groups:
+            if mark:
+                mark(N)
+            st = base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize
+            if N <= 192:
+                rc = lib.gsmi_draw_stamps_f32(st, count, N, nk, ncoef, *o, self.out.data_ptr(), s)
+            else:
+                rc = lib.gsmi_draw_wide_f32(st, count, N, nk, max_ny, ncoef, *o,
+                                            self.scratch.data_ptr(), self.out.data_ptr(), s)
+            _lib.check(rc, "batched stamps (N=%d)" % N)
 
     # -- work-list schedule ----------------------------------------------------------------------
     @staticmethod
@@ -485,8 +497,7 @@ class BatchPlan:
         base = self.dev.data_ptr()
         sc = ctypes.addressof(sched[1])
         if part in ('fold', 'all'):
-            for group in self.stamp_groups:
-                self._launch_stamps(group, s)
+            self._launch_sized(s)
         args_fold = (base + self._o_stamp, self.nrec, sc, base + self._o_ops,
                      base + self._o_leaves,
                      base + self._o_tab)
@@ -639,12 +650,7 @@ class BatchPlan:
             if events:
                 events('end', 0).record()
             return self.out
-        for group in self.stamp_groups:
-            if events:
-                events('fold', group[0]).record()
-            self._launch_stamps(group, s)
-            if events:
-                events('rows', group[0]).record()
+        self._launch_sized(s, (lambda N: events('fold', N).record()) if events else None)
         for N, first, count, max_ny in self.list_groups:
             st = base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize
             if events:

@@ -32,6 +32,7 @@
 #include "../../include/gsmi.h"
 #include "device_program.h"
 #include "launch.h"
+#include "stamp_cells.h"
 
 namespace gsmi {
 namespace {
@@ -62,200 +63,6 @@ template <int N>
 __device__ __forceinline__ constexpr int row_slot(int y)
 {
     return (y % Shape<N>::C1) * Shape<N>::C2 + y / Shape<N>::C1;
-}
-
-// Radix 16 (e^{+2 pi i}) as radix 4 over n1 and radix 4 over n2 with n = 4 n1 + n2, k = k1 + 4 k2.
-__device__ __forceinline__ void bfly16(cplx<float>* v)
-{
-    const float c1 = 0.92387953251128675613f, s1 = 0.38268343236508977173f;   // cos, sin pi/8
-    const float h = 0.70710678118654752440f;
-    cplx<float> a[4][4];
-#pragma unroll
-    for (int n2 = 0; n2 < 4; ++n2) {
-        cplx<float> u[4] = {v[n2], v[n2 + 4], v[n2 + 8], v[n2 + 12]};
-        bfly4(u);
-#pragma unroll
-        for (int k1 = 0; k1 < 4; ++k1) a[n2][k1] = u[k1];
-    }
-    // w16^(n2 k1): w = (c1, s1), w^2 = (h, h), w^3 = (s1, c1), w^4 = i, w^6 = (-h, h),
-    // w^9 = (-c1, -s1)
-    a[1][1] = cmul(a[1][1], cplx<float>{c1, s1});
-    a[1][2] = {h * (a[1][2].x - a[1][2].y), h * (a[1][2].x + a[1][2].y)};
-    a[1][3] = cmul(a[1][3], cplx<float>{s1, c1});
-    a[2][1] = {h * (a[2][1].x - a[2][1].y), h * (a[2][1].x + a[2][1].y)};
-    a[2][2] = {-a[2][2].y, a[2][2].x};
-    a[2][3] = {-h * (a[2][3].x + a[2][3].y), h * (a[2][3].x - a[2][3].y)};
-    a[3][1] = cmul(a[3][1], cplx<float>{s1, c1});
-    a[3][2] = {-h * (a[3][2].x + a[3][2].y), h * (a[3][2].x - a[3][2].y)};
-    a[3][3] = cmul(a[3][3], cplx<float>{-c1, -s1});
-#pragma unroll
-    for (int k1 = 0; k1 < 4; ++k1) {
-        cplx<float> u[4] = {a[0][k1], a[1][k1], a[2][k1], a[3][k1]};
-        bfly4(u);
-#pragma unroll
-        for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = u[k2];
-    }
-}
-
-template <int R>
-__device__ __forceinline__ void bfly(cplx<float>* v)
-{
-    if constexpr (R == 8) bfly8(v);
-    if constexpr (R == 12) bfly12(v);
-    if constexpr (R == 16) bfly16(v);
-}
-
-// Value of leaf l of shape SIG from its quadratic form q = |k'|^2 s^2.
-template <int SIG>
-__device__ __forceinline__ float radial_static(int l, const LeafC<float>& C, const LeafI& I,
-                                               const Tables<float>& tb, float q)
-{
-    const int type = kStaticPrograms[SIG].type[l];
-    if (type == GSMI_LEAF_SERSIC) return C.flux * sersic_f32(C, tb.coef, I.ntab, q);
-    if (type == GSMI_LEAF_MOFFAT) {
-        // eval_leafc's Moffat forms on k = sqrt(q)
-        const float k = sqrtf(fmaxf(q, 0.f));
-        float g, dg;
-        switch (I.kind) {
-          case 1:
-            return C.flux * moffat_trunc_spline<float>(sersic_table<float>(tb, I.aux), I.ntab, q,
-                                                       k, C.p[1], nullptr);
-          case 15: return C.flux * __expf(-k);
-          case 25: return C.flux * __expf(-k) * (1.f + k);
-          case 35: return C.flux * __expf(-k) * (3.f + (3.f + k) * k);
-          case 0: moffat_generic_f32(C, k, &g, &dg); return C.flux * g;
-          default: moffat_int_kind_f32(I.kind, k, &g, &dg); return C.flux * g;
-        }
-    }
-    LeafI J = I;
-    J.type = type;
-    return radial_f32(C, J, tb, q);
-}
-
-// The program at (i dk, m dk) and (i dk, -m dk) of a stamp of shape SIG (real values: radial
-// leaves only).  The last leaf, the PSF, is evaluated once when its form has no kx ky term.
-template <int SIG>
-struct StaticPair {
-    LeafC<float> lr[kProgLeaves];
-    LeafI li[kProgLeaves];
-    Tables<float> tb;
-    float dk;
-    bool even;               // q1 of the last leaf is zero
-
-    __device__ __forceinline__ void operator()(int i, int m, float* p, float* n) const
-    {
-        constexpr int nl = kStaticPrograms[SIG].nl;
-        const float kx = float(i) * dk, ky = float(m) * dk;
-        const float xx = kx * kx, xy = kx * ky, yy = ky * ky;
-        float vp[kProgLeaves] = {}, vn[kProgLeaves] = {};
-#pragma unroll
-        for (int l = 0; l < nl; ++l) {
-            const LeafC<float>& C = lr[l];
-            const float a = C.q0 * xx + C.q2 * yy;
-            if (l == nl - 1) {
-                vp[l] = radial_static<SIG>(l, C, li[l], tb, a + C.q1 * xy);
-                vn[l] = vp[l];
-                if (!even) vn[l] = radial_static<SIG>(l, C, li[l], tb, a - C.q1 * xy);
-            } else {
-                vp[l] = radial_static<SIG>(l, C, li[l], tb, a + C.q1 * xy);
-                vn[l] = radial_static<SIG>(l, C, li[l], tb, a - C.q1 * xy);
-            }
-        }
-        *p = static_ops<float, SIG>(vp, -1, 0.f);
-        *n = static_ops<float, SIG>(vn, -1, 0.f);
-    }
-};
-
-// Fill the packed columns: cell (c, r) of the wrapped grid at buf[c * L + pad(r)], column 0
-// holding cell(0, r) + i cell(N/2, r) (both Hermitian along ky).  hk = Nk/2 < N, so a cell has at
-// most one aliased sample per axis.  X: X(kx), kx <= hk; Y: Y(ky), 0 <= ky <= hk.
-template <int N, typename P>
-__device__ __forceinline__ void fill_cells(const P& pair, int hk, const cplx<float>* X,
-                                           const cplx<float>* Y, cplx<float>* buf)
-{
-    using S = Shape<N>;
-    constexpr int H = N / 2, L = S::L, T = S::T;
-    static_assert(T % H == 0, "a thread keeps one ky");
-    const int tid = threadIdx.x;
-    const int a = N - hk;                    // aliased rows: |ky| from a to N/2
-    const int na = H - a + 1;                // a <= N/2 as Nk >= N
-    // F(i, m) and F(i, -m), m >= 0
-    auto sample = [&](int i, int m, cplx<float>* fp, cplx<float>* fn) {
-        float p, n;
-        pair(i, m, &p, &n);
-        const cplx<float> x = X[i], y = Y[m];
-        const float ac = x.x * y.x, bd = x.y * y.y, ad = x.x * y.y, bc = x.y * y.x;
-        *fp = {p * (ac - bd), p * (ad + bc)};
-        *fn = {n * (ac + bd), n * (bc - ad)};
-    };
-    // primary samples: rows j and N - j, j < N/2 (row N/2 belongs to the next pass)
-    {
-        const int j = tid % H;
-        const int rp = pad<N>(j), rn = pad<N>(N - j);
-        for (int c = tid / H; c < H; c += T / H) {
-            cplx<float> fp, fn;
-            sample(c, j, &fp, &fn);
-            buf[c * L + rp] = fp;
-            if (j) buf[c * L + rn] = fn;
-        }
-    }
-    __syncthreads();
-    const float inv_na = 1.f / float(na);
-    // aliased rows of the columns kx < N/2: ky = N - j adds to row N - j's congruent, -j, and
-    // ky = j - N to row j; row N/2 takes both of ky = +-N/2
-    for (int t = tid; t < H * na; t += T) {
-        const int c = fdiv(t, inv_na);
-        const int j = a + (t - c * na);
-        cplx<float> fp, fn;
-        sample(c, N - j, &fp, &fn);
-        cplx<float>* col = buf + c * L;
-        if (j == H) {
-            col[pad<N>(H)] = cadd(fp, fn);
-        } else {
-            cplx<float>& lo = col[pad<N>(j)];
-            cplx<float>& hi = col[pad<N>(N - j)];
-            lo = cadd(lo, fn);
-            hi = cadd(hi, fp);
-        }
-    }
-    __syncthreads();
-    // columns kx = N/2..hk.  kx > N/2 is congruent to kx - N < 0, whose cells are the
-    // conjugates at -ky of column N - kx; column N/2 itself takes both signs and goes to the
-    // imaginary part of column 0.  wj, wn: the column's folded values at rows j and N - j.
-    auto add_alias = [&](int kx, int j, cplx<float> wj, cplx<float> wn) {
-        const bool nyq = kx == H;
-        cplx<float>* col = buf + (nyq ? 0 : N - kx) * L;
-        cplx<float> dj = cconj(wn), dn = cconj(wj);
-        if (nyq) {
-            const cplx<float> cj = cadd(wj, dj), cn = cadd(wn, dn);
-            dj = {-cj.y, cj.x};
-            dn = {-cn.y, cn.x};
-        }
-        cplx<float>& lo = col[pad<N>(j)];
-        lo = cadd(lo, dj);
-        if (j != 0 && j != H) {
-            cplx<float>& hi = col[pad<N>(N - j)];
-            hi = cadd(hi, dn);
-        }
-    };
-    {
-        const int j = tid % H;
-        for (int kx = H + tid / H; kx <= hk; kx += T / H) {
-            cplx<float> fp, fn;
-            sample(kx, j, &fp, &fn);
-            add_alias(kx, j, fp, fn);
-        }
-    }
-    __syncthreads();
-    for (int t = tid; t < (hk - H + 1) * na; t += T) {
-        const int k = fdiv(t, inv_na);
-        const int j = a + (t - k * na);
-        cplx<float> fp, fn;
-        sample(H + k, N - j, &fp, &fn);
-        if (j == H) fp = fn = cadd(fp, fn);
-        add_alias(H + k, j, fn, fp);
-    }
-    __syncthreads();
 }
 
 // In-place inverse DFT of the H columns: radix C1 over elements C2 apart, the twiddle, then radix
@@ -303,14 +110,6 @@ __device__ __forceinline__ void row_dft(cplx<float>* buf, const cplx<float>* tw,
     constexpr int M = N / 2, L = S::L, T = S::T, R1 = S::R1, R2 = S::R2;
     constexpr int U = R2 / 2;
     const float inv_ny = 1.f / float(ny);
-    // v(c) = E + i O, E = Z(c) + conj Z(M - c), O = (Z(c) - conj Z(M - c)) w^c, and v(M - c) =
-    // conj E + i conj O from the same two inputs
-    auto both = [&](cplx<float> zc, cplx<float> zm, int c, cplx<float>* v, cplx<float>* vm) {
-        const cplx<float> E = {zc.x + zm.x, zc.y - zm.y};
-        const cplx<float> O = cmul(cplx<float>{zc.x - zm.x, zc.y + zm.y}, tw[c]);
-        *v = {E.x - O.y, E.y + O.x};
-        *vm = {E.x + O.y, O.x - E.y};
-    };
     for (int t = threadIdx.x; t < ny * U; t += T) {
         const int u = fdiv(t, inv_ny);
         const int idx = t - u * ny;
@@ -323,22 +122,7 @@ __device__ __forceinline__ void row_dft(cplx<float>* buf, const cplx<float>* tw,
             va[s] = p[(b0 + R2 * s) * L];
             vb[s] = p[(b1 + R2 * s) * L];
         }
-        if (u == 0) {
-            // b = 0: column c pairs with M - c = R2 (R1 - s); column 0 is the packed pair
-            va[0] = {va[0].x + va[0].y, va[0].x - va[0].y};
-#pragma unroll
-            for (int s = 1; s < R1 / 2; ++s)
-                both(va[s], va[R1 - s], R2 * s, &va[s], &va[R1 - s]);
-            cplx<float> dummy;
-            both(va[R1 / 2], va[R1 / 2], M / 2, &va[R1 / 2], &dummy);
-#pragma unroll
-            for (int s = 0; s < R1 / 2; ++s)
-                both(vb[s], vb[R1 - 1 - s], R2 / 2 + R2 * s, &vb[s], &vb[R1 - 1 - s]);
-        } else {
-#pragma unroll
-            for (int s = 0; s < R1; ++s)
-                both(va[s], vb[R1 - 1 - s], b0 + R2 * s, &va[s], &vb[R1 - 1 - s]);
-        }
+        c2r_inputs<R1, R2>(b0, [&](int c) { return tw[c]; }, va, vb);
         bfly<R1>(va);
         bfly<R1>(vb);
 #pragma unroll
@@ -456,7 +240,7 @@ draw_stamp_f32(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
 #pragma unroll
     for (int l = 0; l < kStaticPrograms[SIG].nl; ++l) pair.lr[l] = uniform_leaf(lc[l]);
     pair.even = pair.lr[kStaticPrograms[SIG].nl - 1].q1 == 0.f;
-    fill_cells<N>(pair, hk, X, Y, buf);
+    fill_cells<N, S::L, T>(pair, [](int r) { return pad<N>(r); }, hk, X, Y, 0, H, buf);
     column_dft<N>(buf, tw);
     bool bad = false;
     row_dft<N>(buf, tw, x0, y0, nx, ny, out + st->out_offset, bad);

@@ -377,8 +377,17 @@ int gsmi_rows_list_f32(const gsmi_stamp* stamps, int nstamps, const gsmi_schedul
 int gsmi_draw_stamps_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int max_ncoef,
                          int program, const gsmi_op* ops, const gsmi_leaf* leaves,
                          const double* tables, const float* tables32, float* out, void* stream);
-/* LDS bytes of one workgroup of gsmi_draw_stamps_f32, or -1 for sizes it does not take. */
+/* The same for the larger sizes N = 2^k and 3 2^k from 256 to 4096, through the scratch buffer:
+ * the axis-factor prepass, a kernel over packed columns and one over rows of at most max_ny,
+ * compiled per size.  A stamp that breaks the conditions above has undefined pixels and
+ * GSMI_STAMP_NONFINITE set. */
+int gsmi_draw_wide_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int max_ny,
+                       int max_ncoef, int program, const gsmi_op* ops, const gsmi_leaf* leaves,
+                       const double* tables, const float* tables32, void* scratch, float* out,
+                       void* stream);
+/* LDS bytes of one workgroup of either, or -1 for sizes it does not take. */
 int64_t gsmi_draw_stamps_lds(int N, int max_Nk, int max_ncoef);
+int64_t gsmi_draw_wide_lds(int N, int max_Nk, int max_ncoef);
 
 /* Evaluate a stamp program on a k-image with bounds (xmin..xmin+nx-1, ymin..ymin+ny-1) and
  * spacing dk, writing complex128 values row-major (SBProfile::drawK src/SBProfile.cpp:383-425

@@ -111,3 +111,31 @@ def test_stamp_status_and_rejected_stamps():
     plan.run()
     assert plan.status().tolist() == [0, _lib.STAMP_NONFINITE, 0]
     assert torch.equal(plan.stamp(2), ref[plan.stamp_offset[2]:][:48 * 48].view(48, 48))
+
+
+@pytest.mark.parametrize("gal,psf", [SHAPES[0], SHAPES[3], SHAPES[4], SHAPES[5]])
+@pytest.mark.parametrize("N", [256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096])
+def test_wide_sizes_match_fp64_kernels(gal, psf, N):
+    """The column and row kernels of every larger size, with and without aliased samples: windows
+    of the whole grid, one row, an odd few, and one more than a row chunk."""
+    rng = np.random.default_rng(N + len(gal))
+    for scale in (0.15, 0.28):
+        sides = [(N, N - 1), (N - 2, 1), (N - 1, 33), (17, N - 3)]
+        profs = []
+        for nx, ny in sides:
+            gm, ph = rng.uniform(0., 0.5), rng.uniform(0., np.pi)
+            profs.append(g.Convolve([_gal(gal, 0.4, gm * np.cos(2 * ph), gm * np.sin(2 * ph)),
+                                     _psf(psf, rng.uniform(0.62, 0.9))]))
+        offs = rng.uniform(-0.5, 0.5, (len(sides), 2))
+        nx, ny = np.array(sides).T
+        plan = BatchPlan(profs, nx, ny, scale, offs, precision='f32')
+        assert [x[0] for x in plan.wide_groups] == [N], plan.fft_sizes()
+        plan.out.fill_(float('nan'))
+        plan.run()
+        ref = BatchPlan(profs, nx, ny, scale, offs, precision='f64')
+        ref.run()
+        for i in range(len(sides)):
+            peak = float(ref.stamp(0).abs().max())
+            err = float((plan.stamp(i).double() - ref.stamp(i)).abs().max()) / peak
+            assert err < TOL, (sides[i], scale)
+        assert not plan.status().any()
