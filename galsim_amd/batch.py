@@ -337,6 +337,10 @@ class BatchPlan:
         recs['col_stride'] = (recs['ny'] + 15) // 16 * 16
         rows = recs['col_stride'].astype(np.int64) * (recs['N'].astype(np.int64) // 2 + 1)
         axis = 3 * (recs['Nk'].astype(np.int64) // 2) + 2
+        if precision == 'f64':
+            # room for the leaves of a differentiable batch to grow or shrink fourfold
+            host_leaves, extra = render.moffat_tables(recs, host_leaves, margin=4)
+            axis += extra
         recs['scratch_offset'] = starts(rows)
         recs['axis_offset'] = int(rows.sum()) + starts(axis)
         scratch_need = int(rows.sum() + axis.sum())

@@ -217,6 +217,12 @@ __device__ inline LeafD<T> eval_leafc_d(const LeafC<T>& C, const LeafI& I, const
                     return {g, dg};
                 }
             }
+            if constexpr (sizeof(T) == 8) {
+                LeafD<double> m;
+                if (tb.radial && I.ntab > 0 &&
+                    moffat_table<true>(tb.radial + 2 * size_t(I.aux), ksq, &m.phi, &m.dphi))
+                    return m;
+            }
             LeafD<double> m = moffat_bessel_d(I.kind, rec->p[0] - 1., double(k), double(ksq),
                                               rec->p[1]);
             return {T(m.phi), T(m.dphi)};
@@ -358,6 +364,7 @@ grad_colfft(const gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ o
     const gsmi_leaf* sleaves = leaves + st->leaf_begin;
     const int hk = Nk / 2;
     const cplx<T>* X = scratch + st->axis_offset;
+    if constexpr (sizeof(T) == 8) tb.radial = reinterpret_cast<const double*>(X);
     const cplx<T>* Y = X + hk + 1 + hk;
     const cplx<T>* H = scratch + st->scratch_offset;
     const int ny = st->ny;

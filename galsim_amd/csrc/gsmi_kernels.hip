@@ -28,7 +28,8 @@ namespace gsmi {
 
 
 // ---------------------------------------------------------------------------------------------
-// Kernel 0: per-stamp separable axis factors X(kx), Y(ky) into the workspace (grid: nstamps)
+// Kernel 0: per-stamp separable axis factors X(kx), Y(ky) into the workspace, and in FP64 the
+// tables of its Moffat leaves that have one (grid: nstamps x the workgroups sharing a stamp)
 // ---------------------------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
@@ -36,16 +37,28 @@ axis_factors(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
              const gsmi_leaf* __restrict__ leaves, cplx<T>* __restrict__ ws)
 {
     gsmi_stamp* st = stamps + blockIdx.x;
-    if (threadIdx.x == 0) st->status = 0;         // this launch's status starts clear
+    const int part = blockIdx.y, parts = gridDim.y;
+    // this launch's status starts clear
+    if (threadIdx.x == 0 && part == 0) st->status = 0;
     const int hk = st->Nk / 2;
     const T dk = T(st->dk);
     const gsmi_op* aops = ops + st->op_begin + st->op_count;
     const gsmi_leaf* sleaves = leaves + st->leaf_begin;
     cplx<T>* out = ws + st->axis_offset;
     const int total = (hk + 1) + (2 * hk + 1);
-    for (int e = threadIdx.x; e < total; e += blockDim.x) {
+    for (int e = part * blockDim.x + threadIdx.x; e < total; e += parts * blockDim.x) {
         if (e <= hk) out[e] = axis_factor<T>(aops, st->axis_count, sleaves, T(e) * dk, true);
         else out[e] = axis_factor<T>(aops, st->axis_count, sleaves, T(e - hk - 1 - hk) * dk, false);
+    }
+    if constexpr (sizeof(T) == 8) {
+        for (int o = 0; o < st->op_count; ++o) {
+            const gsmi_op op = ops[st->op_begin + o];
+            if (op.code != GSMI_OP_LEAF) continue;
+            const gsmi_leaf& L = sleaves[op.arg];
+            if (L.type == GSMI_LEAF_MOFFAT && L.kind != 1 && L.ntab > 0)
+                moffat_table_build(L, st->dk, hk, part, parts,
+                                   reinterpret_cast<double*>(out + L.table));
+        }
     }
 }
 
@@ -279,10 +292,12 @@ template <typename T, int SIG = 0>
 __device__ __forceinline__ void fold_item(const gsmi_stamp* __restrict__ st, int first,
                                           int count, int cpg, const gsmi_op* __restrict__ ops,
                                           const gsmi_leaf* __restrict__ leaves,
-                                          const Tables<T>& tb, const cplx<T>* __restrict__ tw,
+                                          Tables<T> tb, const cplx<T>* __restrict__ tw,
                                           int tws, cplx<T>* __restrict__ scratch, cplx<T>* lds,
                                           size_t lds_elems)
 {
+    if constexpr (sizeof(T) == 8)
+        tb.radial = reinterpret_cast<const double*>(scratch + st->axis_offset);
     const int N = st->N;
     const gsmi_op* sops = ops + st->op_begin;
     const int nops = st->op_count;
@@ -1001,8 +1016,10 @@ template <typename T>
 int launch_axis_factors(const gsmi_stamp* stamps, int nstamps, const gsmi_op* ops,
                         const gsmi_leaf* leaves, void* scratch, void* stream)
 {
-    // the kernel also clears each record's status word (the only field a kernel writes)
-    hipLaunchKernelGGL(axis_factors<T>, dim3(nstamps), dim3(kThreads), 0,
+    // the kernel also clears each record's status word (the only field a kernel writes); up to
+    // eight workgroups share a stamp while that gives at most 1024
+    const int parts = nstamps >= 1024 ? 1 : nstamps > 128 ? 1024 / nstamps : 8;
+    hipLaunchKernelGGL(axis_factors<T>, dim3(nstamps, parts), dim3(kThreads), 0,
                        reinterpret_cast<hipStream_t>(stream), const_cast<gsmi_stamp*>(stamps),
                        ops, leaves, reinterpret_cast<cplx<T>*>(scratch));
     return hip_check(hipGetLastError(), "axis_factors launch");

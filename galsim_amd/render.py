@@ -254,6 +254,67 @@ def plan_sizes(prof, bounds):
     return N, Nk, dk
 
 
+def moffat_tables(recs, leaves, margin=0):
+    """Room for the FP64 kernels' radial tables of the untruncated Moffat leaves whose transform
+    is a Bessel function (gsmi_leaf.table / ntab): (leaves with the two fields set, complex values
+    of scratch each stamp of ``recs`` needs after its 3 Nk/2 + 2 axis factors).  The intervals of
+    1/16 octave cover (k rD)^2 from the smallest sample other than 0 to the corner of the k-image,
+    plus ``margin`` octaves for leaves that will move.  Orders above 5 lose digits in the table's
+    recurrence and stay on the Bessel functions."""
+    extra = np.zeros(len(recs), dtype=np.int64)
+    begin = recs['leaf_begin']
+    sel = np.nonzero((leaves['type'] == _lib.LEAF_MOFFAT) &
+                     np.isin(leaves['kind'], (0, 2, 3, 4)) & (leaves['p'][:, 0] <= 6.))[0]
+    if not len(sel) or len(np.unique(begin)) != len(begin):
+        return leaves, extra
+    leaves = leaves.copy()
+    order = np.argsort(begin)
+    L = leaves[sel]
+    pos = np.searchsorted(begin[order], sel, side='right') - 1
+    keep = pos >= 0
+    sel, L, own = sel[keep], L[keep], order[pos[keep]]
+    j = L['jac']
+    a, b = j[:, 0] ** 2 + j[:, 1] ** 2, j[:, 2] ** 2 + j[:, 3] ** 2
+    cross = j[:, 0] * j[:, 2] + j[:, 1] * j[:, 3]
+    big = 0.5 * (a + b) + np.sqrt(0.25 * (a - b) ** 2 + cross ** 2)
+    small = (j[:, 0] * j[:, 3] - j[:, 1] * j[:, 2]) ** 2 / big
+    hk = recs['Nk'][own] / 2.
+    with np.errstate(divide='ignore', invalid='ignore'):
+        octaves = np.log2(2. * hk * hk * big / small)
+    room = np.where(np.isfinite(octaves), np.ceil(16. * (np.minimum(octaves, 64.) + margin)) + 3,
+                    0).astype(np.int64)
+    # one stamp's tables follow one another (leaves of a stamp are consecutive)
+    need = np.where(room > 0, 1 + 6 * room, 0)
+    before = np.cumsum(need) - need
+    first = np.concatenate([[True], own[1:] != own[:-1]]) if len(own) else np.zeros(0, bool)
+    base = np.repeat(before[first], np.diff(np.append(np.nonzero(first)[0], len(own))))
+    axis = 3 * (recs['Nk'][own].astype(np.int64) // 2) + 2
+    leaves['table'][sel] = axis + before - base
+    leaves['ntab'][sel] = room
+    np.add.at(extra, own, need)
+    return leaves, extra
+
+
+def _moffat_room(leaves, Nk):
+    """moffat_tables for the leaf records of one stamp, in plain numbers (the array form costs a
+    single drawing more than its kernels): sets table and ntab, returns the complex values."""
+    extra = 0
+    for rec in leaves:
+        d = rec.d
+        if d['type'] != _lib.LEAF_MOFFAT or d['kind'] not in (0, 2, 3, 4) or d['p'][0] > 6.:
+            continue
+        j0, j1, j2, j3 = d['jac']
+        a, b = j0 * j0 + j1 * j1, j2 * j2 + j3 * j3
+        big = 0.5 * (a + b) + math.hypot(0.5 * (a - b), j0 * j2 + j1 * j3)
+        det = j0 * j3 - j1 * j2
+        ratio = 0.5 * Nk * Nk * big * big / (det * det) if det != 0. else math.inf
+        if 0. < ratio < math.inf:
+            d['table'] = 3 * (Nk // 2) + 2 + extra
+            d['ntab'] = math.ceil(16. * min(math.log2(ratio), 64.)) + 3
+            extra += 1 + 6 * d['ntab']
+    return extra
+
+
 class _Packer:
     """Packs numpy sections into one byte buffer with 256-byte aligned offsets."""
 
@@ -303,6 +364,7 @@ def draw_fft(prof, bounds, precision='f64', return_device=False):
     pk = _Packer()
     o_stamp = pk.add(stamp)
     o_ops = pk.add(ctx.ops_array())
+    extra = _moffat_room(ctx.leaves, Nk) if precision == 'f64' else 0
     o_leaves = pk.add(ctx.leaves_array())
     tables = np.concatenate(ctx.tables) if ctx.tables else np.zeros(1)
     o_tab = pk.add(tables)
@@ -312,7 +374,8 @@ def draw_fft(prof, bounds, precision='f64', return_device=False):
     dev = _device_buffer(torch, pk.host())
     base = dev.data_ptr()
     fdt = torch.float64 if precision == 'f64' else torch.float32
-    scratch = torch.empty((rows + 3 * (Nk // 2) + 2) * 2, dtype=fdt, device='cuda')
+    scratch = torch.empty((rows + 3 * (Nk // 2) + 2 + extra) * 2, dtype=fdt,
+                          device='cuda')
     out = torch.empty((ny, nx), dtype=fdt, device='cuda')
     stream = torch.cuda.current_stream().cuda_stream
     if precision == 'f64':

@@ -131,8 +131,14 @@ typedef struct gsmi_leaf {
     int32_t kind;         /* Moffat: 15,2,25,3,35,4 or 0; 1 = truncated (kV_trunc table,
                              p[0] = beta, p[1] = 1 / knot spacing in k rD); others 0 */
     int32_t table;        /* Sersic, truncated Moffat: offset of its table in the table buffer
-                             (doubles: knots, values, spline second derivatives) */
-    int32_t ntab;         /* Sersic, truncated Moffat: number of knots */
+                             (doubles: knots, values, spline second derivatives).  Moffat of kind
+                             0, 2, 3 or 4 in FP64 with ntab > 0: complex offset, from the stamp's
+                             axis_offset, of 1 + 6 ntab complex values of scratch where the
+                             drawing and adjoint calls keep its radial table */
+    int32_t ntab;         /* Sersic, truncated Moffat: number of knots.  Moffat of kind 0, 2, 3 or
+                             4 in FP64: room for that many intervals of 1/16 octave of (k rD)^2
+                             (samples beyond it, and all with ntab = 0, are evaluated by Bessel
+                             functions one by one) */
     int32_t cliprows;     /* Exponential (FP64): offset of its int2 row ranges, -1 if none;
                              Sersic (FP32): offset (floats, a multiple of 4) in tables32 of its
                              spline as per-interval cubic coefficients (c0, c1, c2, c3) of
