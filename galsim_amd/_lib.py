@@ -153,10 +153,12 @@ _SIGS = {
     'gsmi_fold_list_f32': (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _P]),
     'gsmi_rows_list_f64': (_I, [_P, _I, _P, _P, _P, _P]),
     'gsmi_rows_list_f32': (_I, [_P, _I, _P, _P, _P, _P]),
-    'gsmi_draw_stamps_f32': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P]),
+    'gsmi_draw_stamps_f32': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
+    'gsmi_moffat_tables_f32': (_I, [_P, _I, _P, _P, _P, _P]),
     'gsmi_draw_wide_f32': (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     'gsmi_draw_wide_lds': (ctypes.c_int64, [_I, _I, _I]),
     'gsmi_draw_stamps_lds': (ctypes.c_int64, [_I, _I, _I]),
+    'gsmi_adjoint_stamps_f32': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P]),
     'gsmi_adjoint_partials': (_I, [_I, _I, _P]),
     'gsmi_adjoint_f64': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     'gsmi_adjoint_f32': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P]),

@@ -341,6 +341,15 @@ class BatchPlan:
             # room for the leaves of a differentiable batch to grow or shrink fourfold
             host_leaves, extra = render.moffat_tables(recs, host_leaves, margin=4)
             axis += extra
+        self.program_shape = _program_shape(recs, host_ops, host_leaves)
+        if precision == 'f32' and self.program_shape == 2:
+            # read by the sized kernels; every stamp's region starts on 16 bytes
+            host_leaves, extra = render.moffat_tables(recs, host_leaves, margin=4, kinds=(0,),
+                                                      header=2)
+            axis += axis % 2 + extra
+        self.moffat_tables = precision == 'f32' and bool(
+            np.any((host_leaves['type'] == _lib.LEAF_MOFFAT) & (host_leaves['kind'] == 0) &
+                   (host_leaves['ntab'] > 0)))
         recs['scratch_offset'] = starts(rows)
         recs['axis_offset'] = int(rows.sum()) + starts(axis)
         scratch_need = int(rows.sum() + axis.sum())
@@ -375,7 +384,6 @@ class BatchPlan:
         self._rerun_cleared = np.zeros(n, dtype=bool)
         self.nops = len(host_ops)
         self.nleaves = len(host_leaves)
-        self.program_shape = _program_shape(recs, self.host_ops, self.host_leaves)
         self.stamp_groups, self.wide_groups, self.list_groups = self._split_groups()
         self._sched = None
         self._graph = None
@@ -409,19 +417,34 @@ class BatchPlan:
                 rest.append((N, first, count, max_ny))
         return one, wide, rest
 
+    def sized_program(self):
+        """The program id of the kernels compiled per size: Exponential x Moffat has a second one
+        that reads radial tables."""
+        return 5 if self.moffat_tables else self.program_shape
+
+    def _fill_moffat_tables(self, s):
+        """The FP32 Moffat tables of the records as they are now (the sized kernels read them)."""
+        if self.moffat_tables and (self.stamp_groups or self.wide_groups):
+            base = self.dev.data_ptr()
+            _lib.check(_lib.lib().gsmi_moffat_tables_f32(
+                base + self._o_stamp, self.nrec, base + self._o_ops, base + self._o_leaves,
+                self.scratch.data_ptr(), s), "Moffat tables")
+
     def _launch_sized(self, s, mark=None):
         """The stamp and wide groups' launches on stream ``s``; ``mark(N)``, if given, is called
         before each size's."""
         lib = _lib.lib()
         base = self.dev.data_ptr()
-        o = (self.program_shape, base + self._o_ops, base + self._o_leaves, base + self._o_tab,
+        o = (self.sized_program(), base + self._o_ops, base + self._o_leaves, base + self._o_tab,
              base + self._o_tab32)
+        self._fill_moffat_tables(s)
         for N, first, count, max_ny, nk, ncoef in self.stamp_groups + self.wide_groups:
             if mark:
                 mark(N)
             st = base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize
             if N <= 192:
-                rc = lib.gsmi_draw_stamps_f32(st, count, N, nk, ncoef, *o, self.out.data_ptr(), s)
+                rc = lib.gsmi_draw_stamps_f32(st, count, N, nk, ncoef, *o,
+                                              self.scratch.data_ptr(), self.out.data_ptr(), s)
             else:
                 rc = lib.gsmi_draw_wide_f32(st, count, N, nk, max_ny, ncoef, *o,
                                             self.scratch.data_ptr(), self.out.data_ptr(), s)

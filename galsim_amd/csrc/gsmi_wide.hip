@@ -166,6 +166,7 @@ fold_cols(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
     if constexpr (S::lds_tw)
         for (int e = threadIdx.x; e < N; e += T) twl[e] = twg[e * stride];
     auto tw = [&](int m) { return S::lds_tw ? twl[m] : twg[m * stride]; };
+    tb.radial = scratch + st->axis_offset;
     StaticPair<SIG> pair;
     pair.dk = float(st->dk);
     pair.tb = tb;
@@ -353,6 +354,7 @@ int launch_wide(const gsmi_stamp* stamps, int nstamps, int max_ny, int ncoef, in
       GSMI_WIDE(2)
       GSMI_WIDE(3)
       GSMI_WIDE(4)
+      GSMI_WIDE(5)
 #undef GSMI_WIDE
       default: set_error("gsmi_draw_wide_f32: unknown program shape");
     }

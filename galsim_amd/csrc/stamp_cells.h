@@ -52,6 +52,14 @@ __device__ __forceinline__ void bfly(cplx<float>* v)
     if constexpr (R == 16) bfly16(v);
 }
 
+// Moffat of non-special beta off the table: out of line, as few samples or none take it.
+static __device__ __noinline__ float2 moffat_off_table(const LeafC<float>& C, float k)
+{
+    float g, dg;
+    moffat_generic_f32(C, k, &g, &dg);
+    return {g, dg};
+}
+
 // Value of leaf l of shape SIG from its quadratic form q = |k'|^2 s^2.
 template <int SIG>
 __device__ __forceinline__ float radial_static(int l, const LeafC<float>& C, const LeafI& I,
@@ -70,7 +78,16 @@ __device__ __forceinline__ float radial_static(int l, const LeafC<float>& C, con
           case 15: return C.flux * __expf(-k);
           case 25: return C.flux * __expf(-k) * (1.f + k);
           case 35: return C.flux * __expf(-k) * (3.f + (3.f + k) * k);
-          case 0: moffat_generic_f32(C, k, &g, &dg); return C.flux * g;
+          case 0:
+            // (the out-of-line call costs every kind of a kernel registers: 46 -> 51 us on 1024
+            // stamps of beta = 3, so kernels without tables do without it)
+            if constexpr (SIG == kMoffatTableProgram) {
+                float x;
+                const float4* e = I.ntab > 0 ? moffat_entry(tb.radial + I.aux, q, &x) : nullptr;
+                return C.flux * (e ? moffat_eval(e[0], x) : moffat_off_table(C, k).x);
+            }
+            moffat_generic_f32(C, k, &g, &dg);
+            return C.flux * g;
           default: moffat_int_kind_f32(I.kind, k, &g, &dg); return C.flux * g;
         }
     }

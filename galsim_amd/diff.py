@@ -107,7 +107,13 @@ class DiffPlan:
         lib = _lib.lib()
         need = 1
         self._bins = []
+        # sizes the forward draws by one workgroup per stamp: their adjoint does the same
+        self._stamp_bins = [(N, first, count, nk) for N, first, count, _, nk, _ in
+                            p.stamp_groups]
+        whole = {b[0] for b in self._stamp_bins}
         for N, first, count, max_ny in p.groups:
+            if N in whole:
+                continue
             nd = np.zeros(1, dtype=np.int64)
             _lib.check(lib.gsmi_adjoint_partials(int(N), int(count), _lib.ptr(nd)),
                        "adjoint partials size")
@@ -173,6 +179,16 @@ class DiffPlan:
         o = p.offsets
         s = torch.cuda.current_stream().cuda_stream
         g = self._grad
+        if self._stamp_bins:
+            # the adjoint may follow another set of fields than the last forward's
+            p._fill_moffat_tables(s)
+        for N, first, count, nk in self._stamp_bins:
+            rc = lib.gsmi_adjoint_stamps_f32(
+                base + o['stamp'] + first * _lib.STAMP_DTYPE.itemsize, count, N, nk,
+                p.sized_program(), int(self.shape_gradients), base + o['ops'], base + o['leaves'],
+                base + o['tables'], base + o['tables32'], p.scratch.data_ptr(), resid.data_ptr(),
+                g.data_ptr() + first * NFIELD * 8, s)
+            _lib.check(rc, "adjoint (N=%d)" % N)
         for N, first, count, max_ny, ml, flags in self._bins:
             st = base + o['stamp'] + first * _lib.STAMP_DTYPE.itemsize
             gptr = g.data_ptr() + first * NFIELD * 8

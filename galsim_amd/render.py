@@ -254,17 +254,19 @@ def plan_sizes(prof, bounds):
     return N, Nk, dk
 
 
-def moffat_tables(recs, leaves, margin=0):
-    """Room for the FP64 kernels' radial tables of the untruncated Moffat leaves whose transform
-    is a Bessel function (gsmi_leaf.table / ntab): (leaves with the two fields set, complex values
-    of scratch each stamp of ``recs`` needs after its 3 Nk/2 + 2 axis factors).  The intervals of
+def moffat_tables(recs, leaves, margin=0, kinds=(0, 2, 3, 4), header=1):
+    """Room for the kernels' radial tables of the untruncated Moffat leaves whose transform is a
+    Bessel function (gsmi_leaf.table / ntab): (leaves with the two fields set, complex values of
+    scratch each stamp of ``recs`` needs after its 3 Nk/2 + 2 axis factors).  FP64 tables have a
+    header of one complex value and serve every such kind; FP32 ones have two, start at an even
+    offset, and serve kind 0 (the integer orders have shorter polynomials).  The intervals of
     1/16 octave cover (k rD)^2 from the smallest sample other than 0 to the corner of the k-image,
     plus ``margin`` octaves for leaves that will move.  Orders above 5 lose digits in the table's
     recurrence and stay on the Bessel functions."""
     extra = np.zeros(len(recs), dtype=np.int64)
     begin = recs['leaf_begin']
     sel = np.nonzero((leaves['type'] == _lib.LEAF_MOFFAT) &
-                     np.isin(leaves['kind'], (0, 2, 3, 4)) & (leaves['p'][:, 0] <= 6.))[0]
+                     np.isin(leaves['kind'], kinds) & (leaves['p'][:, 0] <= 6.))[0]
     if not len(sel) or len(np.unique(begin)) != len(begin):
         return leaves, extra
     leaves = leaves.copy()
@@ -284,11 +286,13 @@ def moffat_tables(recs, leaves, margin=0):
     room = np.where(np.isfinite(octaves), np.ceil(16. * (np.minimum(octaves, 64.) + margin)) + 3,
                     0).astype(np.int64)
     # one stamp's tables follow one another (leaves of a stamp are consecutive)
-    need = np.where(room > 0, 1 + 6 * room, 0)
+    need = np.where(room > 0, header + 6 * room, 0)
     before = np.cumsum(need) - need
     first = np.concatenate([[True], own[1:] != own[:-1]]) if len(own) else np.zeros(0, bool)
     base = np.repeat(before[first], np.diff(np.append(np.nonzero(first)[0], len(own))))
     axis = 3 * (recs['Nk'][own].astype(np.int64) // 2) + 2
+    if header == 2:
+        axis += axis % 2
     leaves['table'][sel] = axis + before - base
     leaves['ntab'][sel] = room
     np.add.at(extra, own, need)

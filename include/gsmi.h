@@ -132,13 +132,14 @@ typedef struct gsmi_leaf {
                              p[0] = beta, p[1] = 1 / knot spacing in k rD); others 0 */
     int32_t table;        /* Sersic, truncated Moffat: offset of its table in the table buffer
                              (doubles: knots, values, spline second derivatives).  Moffat of kind
-                             0, 2, 3 or 4 in FP64 with ntab > 0: complex offset, from the stamp's
-                             axis_offset, of 1 + 6 ntab complex values of scratch where the
-                             drawing and adjoint calls keep its radial table */
+                             0, 2, 3 or 4 with ntab > 0: complex offset, from the stamp's
+                             axis_offset, of its radial table in scratch: 1 + 6 ntab complex
+                             values in FP64, filled by the drawing and adjoint calls; 2 + 6 ntab
+                             in FP32, 16-byte aligned, filled by gsmi_moffat_tables_f32 */
     int32_t ntab;         /* Sersic, truncated Moffat: number of knots.  Moffat of kind 0, 2, 3 or
-                             4 in FP64: room for that many intervals of 1/16 octave of (k rD)^2
-                             (samples beyond it, and all with ntab = 0, are evaluated by Bessel
-                             functions one by one) */
+                             4: room for that many intervals of 1/16 octave of (k rD)^2 (samples
+                             beyond it, and all with ntab = 0, are evaluated by Bessel functions
+                             one by one) */
     int32_t cliprows;     /* Exponential (FP64): offset of its int2 row ranges, -1 if none;
                              Sersic (FP32): offset (floats, a multiple of 4) in tables32 of its
                              spline as per-interval cubic coefficients (c0, c1, c2, c3) of
@@ -379,10 +380,12 @@ int gsmi_rows_list_f32(const gsmi_stamp* stamps, int nstamps, const gsmi_schedul
  * included).  Every stamp has N <= Nk <= max_Nk < 2 N, the shape of the nonzero
  * gsmi_schedule.program given and a Sersic table (if the shape has one) with at most max_ncoef
  * coefficient quadruples; a stamp that breaks this is left undrawn with GSMI_STAMP_NONFINITE set.
+ * scratch is read for Moffat tables only (gsmi_moffat_tables_f32) and may be NULL without them.
  * GSMI_E_SIZE for another N or beyond the device's LDS. */
 int gsmi_draw_stamps_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int max_ncoef,
                          int program, const gsmi_op* ops, const gsmi_leaf* leaves,
-                         const double* tables, const float* tables32, float* out, void* stream);
+                         const double* tables, const float* tables32, const void* scratch,
+                         float* out, void* stream);
 /* The same for the larger sizes N = 2^k and 3 2^k from 256 to 4096, through the scratch buffer:
  * the axis-factor prepass, a kernel over packed columns and one over rows of at most max_ny,
  * compiled per size.  A stamp that breaks the conditions above has undefined pixels and
@@ -391,6 +394,11 @@ int gsmi_draw_wide_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk,
                        int max_ncoef, int program, const gsmi_op* ops, const gsmi_leaf* leaves,
                        const double* tables, const float* tables32, void* scratch, float* out,
                        void* stream);
+/* Fill the FP32 tables of every Moffat leaf (kind 0, 2, 3 or 4) with ntab > 0 (gsmi_leaf.table),
+ * which the calls above and gsmi_adjoint_stamps_f32 read for kind 0 where their program is 5
+ * (shape 2 with tables): run it after the records change and before them. */
+int gsmi_moffat_tables_f32(const gsmi_stamp* stamps, int nstamps, const gsmi_op* ops,
+                           const gsmi_leaf* leaves, void* scratch, void* stream);
 /* LDS bytes of one workgroup of either, or -1 for sizes it does not take. */
 int64_t gsmi_draw_stamps_lds(int N, int max_Nk, int max_ncoef);
 int64_t gsmi_draw_wide_lds(int N, int max_Nk, int max_ncoef);
@@ -515,6 +523,15 @@ int gsmi_adjoint_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_ny, i
                      int flags, const gsmi_op* ops, const gsmi_leaf* leaves,
                      const double* tables, const float* tables32, const float* resid,
                      void* scratch, double* partials, double* grad, void* stream);
+
+/* The adjoint of gsmi_draw_stamps_f32: the fields' gradients of nstamps FP32 stamps of one size
+ * N = 128 or 192 and one nonzero program shape (N <= Nk <= max_Nk < 2 N), one workgroup each, with
+ * no scratch and no partials.  shape != 0 computes the Moffat beta derivatives (shape 2).  A stamp
+ * that breaks the conditions gets NaN gradients. */
+int gsmi_adjoint_stamps_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int program,
+                            int shape, const gsmi_op* ops, const gsmi_leaf* leaves,
+                            const double* tables, const float* tables32, const void* scratch,
+                            const float* resid, double* grad, void* stream);
 
 /* -------------------------------------------------------------------------------------------
  * Parameter map of the differentiable Exponential (x) Moffat model (no counterpart in the
