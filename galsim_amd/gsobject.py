@@ -25,6 +25,37 @@ def _real_values(pixels, dtype, add_to_image):
     return vals, float(vals.sum(dtype=float))
 
 
+def _put(image, pixels, add_to_image):
+    if add_to_image:
+        image.array[...] += pixels.astype(image.array.dtype)
+    else:
+        image.array[...] = pixels.astype(image.array.dtype)
+
+
+def _draw_fft_into(prof, image, bounds, precision, add_to_image):
+    """render.draw_fft into an image; returns the flux drawn."""
+    from . import render
+    dest = render.direct_array(image, add_to_image)
+    pixels, added = render.draw_fft(prof, bounds, precision=precision, dest=dest)
+    if dest is None:
+        _put(image, pixels, add_to_image)
+    return added
+
+
+def _draw_real_into(prof, image, bounds, scale, add_to_image):
+    """real.draw_real into an image; returns the flux drawn (_real_values)."""
+    import torch
+    from . import real, render
+    dest = render.direct_array(image, add_to_image)
+    if dest is not None:
+        out = real.draw_real(prof, bounds, scale, device_out=True)
+        return render.store(out.to(torch.float32) if dest.dtype == np.float32 else out, dest)
+    pixels, added = _real_values(real.draw_real(prof, bounds, scale), image.array.dtype,
+                                 add_to_image)
+    _put(image, pixels, add_to_image)
+    return added
+
+
 class GSObject:
     """Base class (galsim/gsobject.py:37-2609).  Subclasses define ``_maxk``, ``_stepk``,
     ``_flux`` and ``_lower(ctx, jac)`` (their contribution to the k-space program)."""
@@ -308,15 +339,9 @@ class GSObject:
         c = image.center
         draw_bounds = image.bounds.shift(PositionI(-c.x, -c.y))
         if use_real:
-            from . import real
-            pixels, added = _real_values(real.draw_real(prof, draw_bounds, 1.0),
-                                         image.array.dtype, add_to_image)
+            added = _draw_real_into(prof, image, draw_bounds, 1.0, add_to_image)
         else:
-            pixels, added = render.draw_fft(prof, draw_bounds, precision=precision)
-        if add_to_image:
-            image.array[...] += pixels.astype(image.array.dtype)
-        else:
-            image.array[...] = pixels.astype(image.array.dtype)
+            added = _draw_fft_into(prof, image, draw_bounds, precision, add_to_image)
         image.added_flux = added / flux_scale
         return image
 
@@ -324,26 +349,13 @@ class GSObject:
         """drawReal (galsim/gsobject.py:1846-1889): the profile sampled at the centre of each
         pixel times the pixel area, its origin at the image's (0, 0), evaluated on the GPU.
         Returns the flux drawn (the sum of the drawn pixel values)."""
-        from . import real
         if image.scale is None or not image.scale > 0:
             raise ValueError("drawReal requires an image with a PixelScale wcs", image)
-        pixels, added = _real_values(real.draw_real(self, image.bounds, float(image.scale)),
-                                     image.array.dtype, add_to_image)
-        if add_to_image:
-            image.array[...] += pixels.astype(image.array.dtype)
-        else:
-            image.array[...] = pixels.astype(image.array.dtype)
-        return added
+        return _draw_real_into(self, image, image.bounds, float(image.scale), add_to_image)
 
     def drawFFT(self, image, add_to_image=False, precision='f64'):
         """drawFFT (galsim/gsobject.py:2014-2045): image bounds centred on the profile origin."""
-        from . import render
-        pixels, added = render.draw_fft(self, image.bounds, precision=precision)
-        if add_to_image:
-            image.array[...] += pixels.astype(image.array.dtype)
-        else:
-            image.array[...] = pixels.astype(image.array.dtype)
-        return added
+        return _draw_fft_into(self, image, image.bounds, precision, add_to_image)
 
     def drawKImage(self, image=None, nx=None, ny=None, bounds=None, scale=None,
                    recenter=True):

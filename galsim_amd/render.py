@@ -333,21 +333,75 @@ class _Packer:
         self.size += (arr.nbytes + _ALIGN - 1) // _ALIGN * _ALIGN
         return off
 
-    def host(self):
-        buf = np.zeros(max(self.size, _ALIGN), dtype=np.uint8)
+    def write(self, buf):
         for off, b in self.parts:
             buf[off:off + len(b)] = b
+
+    def host(self):
+        buf = np.zeros(max(self.size, _ALIGN), dtype=np.uint8)
+        self.write(buf)
         return buf
 
 
-def _device_buffer(torch, host_bytes):
-    t = torch.from_numpy(host_bytes)
-    return t.to('cuda', non_blocking=False)
+STAGE_BYTES = 4 << 20          # one of the two pinned blocks a device-to-host copy goes through
+DEVICE_SUM = 65536             # pixels from which the flux is summed on the device
 
 
-def draw_fft(prof, bounds, precision='f64', return_device=False):
+def direct_array(image, add_to_image):
+    """The image's array if drawn pixels can be stored straight into it, else None."""
+    a = image.array
+    ok = not add_to_image and a.dtype in (np.float32, np.float64) and a.flags.c_contiguous and \
+        a.flags.writeable and a.dtype.isnative
+    return a if ok else None
+
+
+def store(t, dest):
+    """Copy a contiguous device tensor into a C-contiguous float array of its shape, converting,
+    and return the sum of the tensor's values in double.
+
+    The rows come through two pinned blocks of at most STAGE_BYTES, one filled by the device while
+    the other is written out.  A copy to pageable memory is staged by the runtime anyway, into an
+    array that is then converted and copied twice more: a 1024 x 1000 FP64 image took 0.93 ms that
+    way and 0.23 ms this way.  Summing a large image on the host costs more than a device kernel
+    (0.12 ms against 0.03 ms at that size, 2 us against 20 us at 64 x 64)."""
+    import torch
+    flat, out = t.reshape(-1), torch.from_numpy(dest.reshape(-1))
+    n = flat.numel()
+    total = flat.sum(dtype=torch.float64) if n >= DEVICE_SUM else None
+    step = STAGE_BYTES // t.element_size()
+    spans = [(a, min(a + step, n)) for a in range(0, n, step)]
+    blocks = [torch.empty(min(step, n), dtype=t.dtype, pin_memory=True)
+              for _ in range(min(2, len(spans)))]
+    ready = [torch.cuda.Event() for _ in blocks]
+
+    def fetch(k):
+        a, b = spans[k]
+        blocks[k % 2][:b - a].copy_(flat[a:b], non_blocking=True)
+        ready[k % 2].record()
+
+    for k in range(len(blocks)):
+        fetch(k)
+    for k, (a, b) in enumerate(spans):
+        ready[k % 2].synchronize()
+        out[a:b].copy_(blocks[k % 2][:b - a])
+        if k + 2 < len(spans):
+            fetch(k + 2)
+    if total is not None:
+        return float(total)
+    return float(blocks[0].numpy().sum(dtype=float)) if n else 0.
+
+
+def _device_buffer(torch, packer):
+    """The packed sections on the device: written into pinned memory, copied without a wait."""
+    host = torch.empty(max(packer.size, _ALIGN), dtype=torch.uint8, pin_memory=True)
+    packer.write(host.numpy())
+    return host.to('cuda', non_blocking=True)
+
+
+def draw_fft(prof, bounds, precision='f64', return_device=False, dest=None):
     """Render ``prof`` (already in image coordinates) onto ``bounds`` (centred on the profile
-    origin, as drawFFT expects).  Returns (pixels, added_flux)."""
+    origin, as drawFFT expects).  Returns (pixels, added_flux); with ``dest`` (a C-contiguous
+    float array of the bounds' shape) the pixels are stored there and ``dest`` is returned."""
     if precision not in ('f64', 'f32'):
         raise ValueError("precision must be 'f64' or 'f32'")
     lib = _lib.lib()
@@ -375,7 +429,7 @@ def draw_fft(prof, bounds, precision='f64', return_device=False):
     o_tab32 = pk.add(ctx.tables32_array())
     clip = np.concatenate(ctx.clip) if ctx.clip else np.zeros(2, dtype=np.int32)
     o_clip = pk.add(clip)
-    dev = _device_buffer(torch, pk.host())
+    dev = _device_buffer(torch, pk)
     base = dev.data_ptr()
     fdt = torch.float64 if precision == 'f64' else torch.float32
     scratch = torch.empty((rows + 3 * (Nk // 2) + 2 + extra) * 2, dtype=fdt,
@@ -388,7 +442,7 @@ def draw_fft(prof, bounds, precision='f64', return_device=False):
                                    out.data_ptr(), stream)
         if rc == -5:
             # an FFT size beyond the fused kernels' LDS: the same steps unfused on the GPU
-            return _draw_fft_unfused(prof, bounds, N, Nk, dk, return_device)
+            return _draw_fft_unfused(prof, bounds, N, Nk, dk, return_device, dest)
     else:
         rc = lib.gsmi_draw_fft_f32(base + o_stamp, 1, N, ny, base + o_ops, base + o_leaves,
                                    base + o_tab, base + o_tab32, scratch.data_ptr(),
@@ -396,11 +450,13 @@ def draw_fft(prof, bounds, precision='f64', return_device=False):
     _lib.check(rc, "gsmi_draw_fft_%s" % precision)
     if return_device:
         return out, (dev, scratch)
+    if dest is not None:
+        return dest, store(out, dest)
     host = out.cpu().numpy()
     return host, float(host.sum(dtype=float))
 
 
-def _draw_fft_unfused(prof, bounds, N, Nk, dk, return_device=False):
+def _draw_fft_unfused(prof, bounds, N, Nk, dk, return_device=False, dest=None):
     """drawFFT in FP64 as the reference's separate steps, for FFT sizes whose column transform
     does not fit one workgroup's LDS (N = 6144, 8192): the k-image on (0..Nk/2, -Nk/2..Nk/2)
     (gsmi_draw_kimage_f64, with the reference's clip rows), wrapImage(hermx) onto the N-grid
@@ -419,7 +475,7 @@ def _draw_fft_unfused(prof, bounds, N, Nk, dk, return_device=False):
     o_tab = pk.add(tables)
     clip = np.concatenate(ctx.clip) if ctx.clip else np.zeros(2, dtype=np.int32)
     o_clip = pk.add(clip)
-    dev = _device_buffer(torch, pk.host())
+    dev = _device_buffer(torch, pk)
     base = dev.data_ptr()
     stream = torch.cuda.current_stream().cuda_stream
     h = Nk // 2
@@ -440,6 +496,8 @@ def _draw_fft_unfused(prof, bounds, N, Nk, dk, return_device=False):
                bounds.xmin + N // 2: bounds.xmax + N // 2 + 1].contiguous()
     if return_device:
         return out, (dev,)
+    if dest is not None:
+        return dest, store(out, dest)
     host = out.cpu().numpy()
     return host, float(host.sum(dtype=float))
 
@@ -469,7 +527,7 @@ def draw_kimage(prof, bounds, dk, jac=None, Nk=None, return_device=False):
     o_tab = pk.add(tables)
     clip = np.concatenate(ctx.clip) if ctx.clip else np.zeros(2, dtype=np.int32)
     o_clip = pk.add(clip)
-    dev = _device_buffer(torch, pk.host())
+    dev = _device_buffer(torch, pk)
     base = dev.data_ptr()
     out = torch.empty((ny, nx, 2), dtype=torch.float64, device='cuda')
     rc = lib.gsmi_draw_kimage_f64(base + o_ops, len(ctx.ops), base + o_leaves, base + o_tab,
@@ -497,7 +555,7 @@ def kvalue(prof, kx, ky):
     o_leaves = pk.add(ctx.leaves_array())
     tables = np.concatenate(ctx.tables) if ctx.tables else np.zeros(1)
     o_tab = pk.add(tables)
-    dev = _device_buffer(torch, pk.host())
+    dev = _device_buffer(torch, pk)
     base = dev.data_ptr()
     out = torch.empty(2, dtype=torch.float64, device='cuda')
     rc = lib.gsmi_draw_kimage_f64(base + o_ops, len(ctx.ops), base + o_leaves, base + o_tab,
