@@ -156,6 +156,8 @@ _SIGS = {
     'gsmi_draw_stamps_f32': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     'gsmi_moffat_tables_f32': (_I, [_P, _I, _P, _P, _P, _P]),
     'gsmi_draw_wide_f32': (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
+    'gsmi_draw_wide_f64': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
+    'gsmi_draw_wide_lds_f64': (ctypes.c_int64, [_I, _I]),
     'gsmi_draw_wide_lds': (ctypes.c_int64, [_I, _I, _I]),
     'gsmi_draw_stamps_lds': (ctypes.c_int64, [_I, _I, _I]),
     'gsmi_adjoint_stamps_f32': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P]),

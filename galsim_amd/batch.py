@@ -390,18 +390,19 @@ class BatchPlan:
         self.tuning = None
 
     def _split_groups(self):
-        """(stamp groups, wide groups, list groups): how each FFT size is drawn.  FP32 batches of
-        a specialised program shape whose stamps have Nk < 2 N (at most one alias per axis, which
-        is what the cell passes of these kernels add) take the kernels compiled per size: one
+        """(stamp groups, wide groups, list groups): how each FFT size is drawn.  Batches of a
+        specialised program shape whose stamps have Nk < 2 N (at most one alias per axis, which is
+        what the cell passes of these kernels add) take the kernels compiled per size: in FP32 one
         workgroup per stamp at N = 128 and 192, whose wrapped grid fits its LDS
-        (gsmi_draw_stamps_f32), a column and a row kernel from 256 to 4096 (gsmi_draw_wide_f32);
-        both (N, first, count, max_ny, largest Nk, Sersic coefficients).  Everything else, as
+        (gsmi_draw_stamps_f32), and a column and a row kernel from 256 to 4096
+        (gsmi_draw_wide_f32); in FP64 those two from 128 to 2048 (gsmi_draw_wide_f64); each
+        (N, first, count, max_ny, largest Nk, Sersic coefficients).  Everything else, as
         (N, first, count, max_ny), takes the fold and row kernels of any shape and size."""
-        if self.precision != 'f32' or not self.program_shape:
+        if not self.program_shape:
             return [], [], list(self.groups)
         ncoef = 0
         sel = self.host_leaves['type'] == _lib.LEAF_SERSIC
-        if sel.any():
+        if sel.any() and self.precision == 'f32':
             if np.any(self.host_leaves['cliprows'][sel] < 0):
                 return [], [], list(self.groups)
             ncoef = int(self.host_leaves['ntab'][sel].max()) - 1
@@ -409,7 +410,11 @@ class BatchPlan:
         lib = _lib.lib()
         for N, first, count, max_ny in self.groups:
             nk = int(self.recs['Nk'][first:first + count].max())
-            if 0 < lib.gsmi_draw_stamps_lds(N, nk, ncoef) <= LIST_LDS_LIMIT:
+            if self.precision == 'f64':
+                fits = 0 < lib.gsmi_draw_wide_lds_f64(N, nk) <= LIST_LDS_LIMIT
+                (wide if fits else rest).append((N, first, count, max_ny, nk, 0) if fits else
+                                                (N, first, count, max_ny))
+            elif 0 < lib.gsmi_draw_stamps_lds(N, nk, ncoef) <= LIST_LDS_LIMIT:
                 one.append((N, first, count, max_ny, nk, ncoef))
             elif 0 < lib.gsmi_draw_wide_lds(N, nk, ncoef) <= LIST_LDS_LIMIT:
                 wide.append((N, first, count, max_ny, nk, ncoef))
@@ -436,13 +441,16 @@ class BatchPlan:
         lib = _lib.lib()
         base = self.dev.data_ptr()
         o = (self.sized_program(), base + self._o_ops, base + self._o_leaves, base + self._o_tab,
-             base + self._o_tab32)
+             base + (self._o_tab32 if self.precision == 'f32' else self._o_clip))
         self._fill_moffat_tables(s)
         for N, first, count, max_ny, nk, ncoef in self.stamp_groups + self.wide_groups:
             if mark:
                 mark(N)
             st = base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize
-            if N <= 192:
+            if self.precision == 'f64':
+                rc = lib.gsmi_draw_wide_f64(st, count, N, nk, max_ny, *o,
+                                            self.scratch.data_ptr(), self.out.data_ptr(), s)
+            elif N <= 192:
                 rc = lib.gsmi_draw_stamps_f32(st, count, N, nk, ncoef, *o,
                                               self.scratch.data_ptr(), self.out.data_ptr(), s)
             else:

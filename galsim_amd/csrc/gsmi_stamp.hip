@@ -226,7 +226,9 @@ draw_stamp_f32(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
         }
     }
     tb.radial = scratch + st->axis_offset;
-    StaticPair<SIG> pair;
+    StaticPair<float, SIG> pair;
+    pair.leaves = sleaves;
+    pair.Nk = st->Nk;
     pair.dk = dk;
     pair.tb = tb;
     if (int(threadIdx.x) < kStaticPrograms[SIG].nl)

@@ -319,6 +319,22 @@ def _moffat_room(leaves, Nk):
     return extra
 
 
+_STATIC_BY_OPS = {}
+for _sid, (_sops, _types) in _lib.STATIC_PROGRAMS.items():
+    _STATIC_BY_OPS.setdefault(_sops, []).append((_sid, _types))
+
+
+def _static_program(ctx, nops):
+    """The specialised program shape of a lowered stamp, or 0."""
+    if nops > 5:
+        return 0
+    prog = tuple((int(op[0]), int(op[1])) for op in ctx.ops[:nops])
+    for sid, types in _STATIC_BY_OPS.get(prog, ()):
+        if all(ctx.leaves[l].d['type'] == t for l, t in enumerate(types)):
+            return sid
+    return 0
+
+
 class _Packer:
     """Packs numpy sections into one byte buffer with 256-byte aligned offsets."""
 
@@ -436,7 +452,13 @@ def draw_fft(prof, bounds, precision='f64', return_device=False, dest=None):
                           device='cuda')
     out = torch.empty((ny, nx), dtype=fdt, device='cuda')
     stream = torch.cuda.current_stream().cuda_stream
-    if precision == 'f64':
+    program = _static_program(ctx, nops) if precision == 'f64' else 0
+    if program and lib.gsmi_draw_wide_lds_f64(N, Nk) > 0:
+        # (the specialised kernels' tiles are below any gfx950 limit: 107 KB of LDS at most)
+        rc = lib.gsmi_draw_wide_f64(base + o_stamp, 1, N, Nk, ny, program, base + o_ops,
+                                    base + o_leaves, base + o_tab, base + o_clip,
+                                    scratch.data_ptr(), out.data_ptr(), stream)
+    elif precision == 'f64':
         rc = lib.gsmi_draw_fft_f64(base + o_stamp, 1, N, ny, base + o_ops, base + o_leaves,
                                    base + o_tab, base + o_clip, scratch.data_ptr(),
                                    out.data_ptr(), stream)

@@ -394,14 +394,20 @@ int gsmi_draw_wide_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk,
                        int max_ncoef, int program, const gsmi_op* ops, const gsmi_leaf* leaves,
                        const double* tables, const float* tables32, void* scratch, float* out,
                        void* stream);
+/* The FP64 form, N = 2^k and 3 2^k from 128 to 2048, programs 1 to 4. */
+int gsmi_draw_wide_f64(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int max_ny,
+                       int program, const gsmi_op* ops, const gsmi_leaf* leaves,
+                       const double* tables, const int32_t* cliprows, void* scratch, double* out,
+                       void* stream);
 /* Fill the FP32 tables of every Moffat leaf (kind 0, 2, 3 or 4) with ntab > 0 (gsmi_leaf.table),
  * which the calls above and gsmi_adjoint_stamps_f32 read for kind 0 where their program is 5
  * (shape 2 with tables): run it after the records change and before them. */
 int gsmi_moffat_tables_f32(const gsmi_stamp* stamps, int nstamps, const gsmi_op* ops,
                            const gsmi_leaf* leaves, void* scratch, void* stream);
-/* LDS bytes of one workgroup of either, or -1 for sizes it does not take. */
+/* LDS bytes of one workgroup of each, or -1 for sizes it does not take. */
 int64_t gsmi_draw_stamps_lds(int N, int max_Nk, int max_ncoef);
 int64_t gsmi_draw_wide_lds(int N, int max_Nk, int max_ncoef);
+int64_t gsmi_draw_wide_lds_f64(int N, int max_Nk);
 
 /* Evaluate a stamp program on a k-image with bounds (xmin..xmin+nx-1, ymin..ymin+ny-1) and
  * spacing dk, writing complex128 values row-major (SBProfile::drawK src/SBProfile.cpp:383-425

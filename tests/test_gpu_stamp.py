@@ -31,6 +31,13 @@ def _psf(kind, fwhm):
     return g.Kolmogorov(fwhm=fwhm)
 
 
+def _general(plan):
+    """The plan drawn by the fold and row kernels of any shape and size."""
+    plan.stamp_groups, plan.wide_groups, plan.list_groups = [], [], list(plan.groups)
+    plan.run()
+    return plan
+
+
 def _peak_rel(a, b):
     return float((a.double() - b.double()).abs().max() / b.double().abs().max())
 
@@ -58,11 +65,8 @@ def test_stamps_match_fp64_and_list_kernels(gal, psf, scale):
     assert {x[0] for x in plan.stamp_groups} <= {128, 192} and plan.stamp_groups
     plan.out.fill_(float('nan'))
     plan.run()
-    lists = BatchPlan(profs, nx, ny, scale, offs, precision='f32')
-    lists.stamp_groups, lists.list_groups = [], list(lists.groups)
-    lists.run()
-    ref = BatchPlan(profs, nx, ny, scale, offs, precision='f64')
-    ref.run()
+    lists = _general(BatchPlan(profs, nx, ny, scale, offs, precision='f32'))
+    ref = _general(BatchPlan(profs, nx, ny, scale, offs, precision='f64'))
     for i in range(len(sides)):
         assert _peak_rel(plan.stamp(i), ref.stamp(i)) < TOL, (sides[i], plan.recs['Nk'])
         assert _peak_rel(plan.stamp(i), lists.stamp(i)) < TOL, sides[i]
@@ -76,6 +80,8 @@ def test_stamp_path_is_left_for_other_sizes_and_shapes():
     e, m = g.Exponential(half_light_radius=0.4), g.Moffat(beta=3, fwhm=0.7)
     assert plan(g.Convolve([e, m])).stamp_groups
     assert not plan(g.Convolve([e, m]), precision='f64').stamp_groups
+    assert plan(g.Convolve([e, m]), precision='f64').wide_groups
+    assert not plan(g.Convolve([e, m, g.Gaussian(sigma=0.1)]), precision='f64').wide_groups
     assert not plan(g.Convolve([e, m, g.Gaussian(sigma=0.1)])).stamp_groups
     assert not plan(g.Convolve([e.shift(0.1, 0.2), m])).stamp_groups
     coarse = plan(g.Convolve([e, m]), scale=0.9)
@@ -132,10 +138,42 @@ def test_wide_sizes_match_fp64_kernels(gal, psf, N):
         assert [x[0] for x in plan.wide_groups] == [N], plan.fft_sizes()
         plan.out.fill_(float('nan'))
         plan.run()
-        ref = BatchPlan(profs, nx, ny, scale, offs, precision='f64')
-        ref.run()
+        ref = _general(BatchPlan(profs, nx, ny, scale, offs, precision='f64'))
         for i in range(len(sides)):
             peak = float(ref.stamp(0).abs().max())
             err = float((plan.stamp(i).double() - ref.stamp(i)).abs().max()) / peak
             assert err < TOL, (sides[i], scale)
+        assert not plan.status().any()
+
+
+@pytest.mark.parametrize("gal,psf", SHAPES)
+@pytest.mark.parametrize("N", [128, 192, 256, 384, 512, 768, 1024, 1536, 2048])
+def test_wide_fp64_matches_general_kernels(gal, psf, N):
+    """The FP64 column and row kernels, samples beside the Exponential's clip rows included, in a
+    batch and (a window of one shape) through drawImage."""
+    rng = np.random.default_rng(N + len(psf))
+    for scale in (0.15, 0.23):
+        sides = [(N, N - 1), (N - 2, 1), (N - 1, 33), (17, N - 3)]
+        profs = []
+        for i, (nx, ny) in enumerate(sides):
+            gm, ph = rng.uniform(0., 0.5), rng.uniform(0., np.pi)
+            p = _psf(psf, rng.uniform(0.62, 0.9))
+            if i == 1:
+                p = p.shear(g1=0.1, g2=-0.15)
+            hlr = 0.12 if N <= 192 else 0.4
+            profs.append(g.Convolve([_gal(gal, hlr, gm * np.cos(2 * ph), gm * np.sin(2 * ph)),
+                                     p]))
+        offs = rng.uniform(-0.5, 0.5, (len(sides), 2))
+        nx, ny = np.array(sides).T
+        plan = BatchPlan(profs, nx, ny, scale, offs, precision='f64')
+        assert [x[0] for x in plan.wide_groups] == [N], plan.fft_sizes()
+        plan.out.fill_(float('nan'))
+        plan.run()
+        ref = _general(BatchPlan(profs, nx, ny, scale, offs, precision='f64'))
+        for i in range(len(sides)):
+            assert _peak_rel(plan.stamp(i), ref.stamp(i)) < 2e-14, (sides[i], scale)
+        one = profs[3].drawImage(nx=17, ny=N - 3, scale=scale, offset=tuple(offs[3]),
+                                 dtype=np.float64).array
+        b = ref.stamp(3).cpu().numpy()
+        assert np.abs(one - b).max() < 2e-14 * np.abs(b).max()
         assert not plan.status().any()
