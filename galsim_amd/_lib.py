@@ -68,6 +68,12 @@ class Schedule(ctypes.Structure):
                 ('program', ctypes.c_int32)]
 
 
+class SizeGroup(ctypes.Structure):
+    """gsmi_size_group: the stamps of one FFT size."""
+    _fields_ = [('N', ctypes.c_int32), ('first', ctypes.c_int32), ('count', ctypes.c_int32),
+                ('max_ny', ctypes.c_int32), ('max_Nk', ctypes.c_int32)]
+
+
 # Program shapes with specialised fold kernels (gsmi_schedule.program): post-order ops
 # ((code, arg), ...) and the leaf type of each slot.
 STATIC_PROGRAMS = {
@@ -155,8 +161,8 @@ _SIGS = {
     'gsmi_rows_list_f32': (_I, [_P, _I, _P, _P, _P, _P]),
     'gsmi_draw_stamps_f32': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     'gsmi_moffat_tables_f32': (_I, [_P, _I, _P, _P, _P, _P]),
-    'gsmi_draw_wide_f32': (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
-    'gsmi_draw_wide_f64': (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
+    'gsmi_draw_wide_f32': (_I, [_P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
+    'gsmi_draw_wide_f64': (_I, [_P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     'gsmi_draw_wide_lds_f64': (ctypes.c_int64, [_I, _I]),
     'gsmi_draw_wide_lds': (ctypes.c_int64, [_I, _I, _I]),
     'gsmi_draw_stamps_lds': (ctypes.c_int64, [_I, _I, _I]),

@@ -443,20 +443,28 @@ class BatchPlan:
         o = (self.sized_program(), base + self._o_ops, base + self._o_leaves, base + self._o_tab,
              base + (self._o_tab32 if self.precision == 'f32' else self._o_clip))
         self._fill_moffat_tables(s)
-        for N, first, count, max_ny, nk, ncoef in self.stamp_groups + self.wide_groups:
+        for N, first, count, max_ny, nk, ncoef in self.stamp_groups:
             if mark:
                 mark(N)
-            st = base + self._o_stamp + first * _lib.STAMP_DTYPE.itemsize
-            if self.precision == 'f64':
-                rc = lib.gsmi_draw_wide_f64(st, count, N, nk, max_ny, *o,
-                                            self.scratch.data_ptr(), self.out.data_ptr(), s)
-            elif N <= 192:
-                rc = lib.gsmi_draw_stamps_f32(st, count, N, nk, ncoef, *o,
-                                              self.scratch.data_ptr(), self.out.data_ptr(), s)
-            else:
-                rc = lib.gsmi_draw_wide_f32(st, count, N, nk, max_ny, ncoef, *o,
-                                            self.scratch.data_ptr(), self.out.data_ptr(), s)
+            rc = lib.gsmi_draw_stamps_f32(base + self._o_stamp +
+                                          first * _lib.STAMP_DTYPE.itemsize, count, N, nk, ncoef,
+                                          *o, self.scratch.data_ptr(), self.out.data_ptr(), s)
             _lib.check(rc, "batched stamps (N=%d)" % N)
+        # all sizes in one call, unless each is to be marked
+        for groups in ([[g] for g in self.wide_groups] if mark else [self.wide_groups]):
+            if not groups:
+                continue
+            if mark:
+                mark(groups[0][0])
+            arr = (_lib.SizeGroup * len(groups))(*[g[:5] for g in groups])
+            args = (base + self._o_stamp, ctypes.addressof(arr), len(groups))
+            if self.precision == 'f64':
+                rc = lib.gsmi_draw_wide_f64(*args, *o, self.scratch.data_ptr(),
+                                            self.out.data_ptr(), s)
+            else:
+                rc = lib.gsmi_draw_wide_f32(*args, groups[0][5], *o, self.scratch.data_ptr(),
+                                            self.out.data_ptr(), s)
+            _lib.check(rc, "batched stamps (N=%d...)" % groups[0][0])
 
     # -- work-list schedule ----------------------------------------------------------------------
     @staticmethod
@@ -531,8 +539,6 @@ class BatchPlan:
         lib = _lib.lib()
         base = self.dev.data_ptr()
         sc = ctypes.addressof(sched[1])
-        if part in ('fold', 'all'):
-            self._launch_sized(s)
         args_fold = (base + self._o_stamp, self.nrec, sc, base + self._o_ops,
                      base + self._o_leaves,
                      base + self._o_tab)
@@ -544,6 +550,9 @@ class BatchPlan:
                 rc = lib.gsmi_fold_list_f64(*args_fold, base + self._o_clip,
                                             self.scratch.data_ptr(), s)
             _lib.check(rc, "fold work list")
+        if part in ('fold', 'all'):
+            # after the list's prepass, which clears the status of every stamp
+            self._launch_sized(s)
         if part in ('rows', 'all') and self.list_groups:
             f = lib.gsmi_rows_list_f32 if self.precision == 'f32' else lib.gsmi_rows_list_f64
             rc = f(base + self._o_stamp, self.nrec, sc, self.scratch.data_ptr(),

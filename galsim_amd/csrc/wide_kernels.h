@@ -150,16 +150,16 @@ constexpr size_t rows_lds = sizeof(cplx<F>) * size_t(Rows<F, N>::R) * Rows<F, N>
 
 // Grid: (ceil(N/2 / (CC per_wg)), stamps): per_wg chunks of CC columns each.  A stamp the launch
 // cannot draw is flagged and its scratch left as it was.
-template <typename F, int N, int SIG>
-__global__ void __launch_bounds__((Cols<F, N>::T), (Cols<F, N>::WAVES))
-fold_cols(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
-          const gsmi_leaf* __restrict__ leaves, Tables<F> tb, TwiddleSet<F> tws,
-          int lds_bytes, int per_wg, cplx<F>* __restrict__ scratch)
+template <typename F, int N, int SIG, int T>
+__device__ __forceinline__ void fold_cols_body(gsmi_stamp* __restrict__ st, int block,
+                                               const gsmi_op* __restrict__ ops,
+                                               const gsmi_leaf* __restrict__ leaves, Tables<F> tb,
+                                               TwiddleSet<F> tws, int lds_bytes, int per_wg,
+                                               cplx<F>* __restrict__ scratch)
 {
     using S = Cols<F, N>;
-    constexpr int H = N / 2, T = S::T, CC = S::CC;
+    constexpr int H = N / 2, CC = S::CC;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    gsmi_stamp* st = stamps + blockIdx.y;
     const int hk = st->Nk / 2;
     const gsmi_op* sops = ops + st->op_begin;
     const gsmi_leaf* sleaves = leaves + st->leaf_begin;
@@ -211,8 +211,8 @@ fold_cols(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
     const size_t cs = col_stride(st);
     cplx<F>* out = scratch + st->scratch_offset;
     const float inv_ny = 1.f / float(ny);
-    const int cend = min(H, int(blockIdx.x + 1) * per_wg * CC);
-    for (int c0 = blockIdx.x * per_wg * CC; c0 < cend; c0 += CC) {
+    const int cend = min(H, (block + 1) * per_wg * CC);
+    for (int c0 = block * per_wg * CC; c0 < cend; c0 += CC) {
         fill_cells<N, S::L, T>(pair, [](int r) { return S::pad(r); }, hk, X, Y, c0, CC, buf);
         for (int t = threadIdx.x; t < CC * S::NB; t += T) {
             const int cl = unsigned(t) / unsigned(S::NB);
@@ -261,18 +261,26 @@ fold_cols(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
     }
 }
 
-// Grid: (ceil(max ny / R), stamps).
-template <typename F, int N>
-__global__ void __launch_bounds__((Rows<F, N>::T), (Rows<F, N>::WAVES))
-row_pixels(gsmi_stamp* __restrict__ stamps, const cplx<F>* __restrict__ scratch,
-           TwiddleSet<F> tws, F* __restrict__ out)
+template <typename F, int N, int SIG>
+__global__ void __launch_bounds__((Cols<F, N>::T), (Cols<F, N>::WAVES))
+fold_cols(gsmi_stamp* __restrict__ stamps, const gsmi_op* __restrict__ ops,
+          const gsmi_leaf* __restrict__ leaves, Tables<F> tb, TwiddleSet<F> tws,
+          int lds_bytes, int per_wg, cplx<F>* __restrict__ scratch)
+{
+    fold_cols_body<F, N, SIG, Cols<F, N>::T>(stamps + blockIdx.y, blockIdx.x, ops, leaves, tb, tws,
+                                             lds_bytes, per_wg, scratch);
+}
+
+template <typename F, int N, int T>
+__device__ __forceinline__ void row_pixels_body(gsmi_stamp* __restrict__ st, int block,
+                                                const cplx<F>* __restrict__ scratch,
+                                                TwiddleSet<F> tws, F* __restrict__ out)
 {
     using S = Rows<F, N>;
-    constexpr int M = N / 2, T = S::T, R = S::R, Q = S::NB, U = Q / 2, D1 = S::C1;
+    constexpr int M = N / 2, R = S::R, Q = S::NB, U = Q / 2, D1 = S::C1;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cplx<F>* buf = reinterpret_cast<cplx<F>*>(smem_raw);
-    gsmi_stamp* st = stamps + blockIdx.y;
-    const int r0 = blockIdx.x * R;
+    const int r0 = block * R;
     const int nx = st->nx, x0 = st->x0;
     const int nrow = min(R, st->ny - r0);
     if (st->N != N || nrow <= 0 || x0 < -M || x0 + nx > M) return;
@@ -343,6 +351,86 @@ row_pixels(gsmi_stamp* __restrict__ stamps, const cplx<F>* __restrict__ scratch,
     if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(&st->status, GSMI_STAMP_NONFINITE);
 }
 
+// Grid: (ceil(max ny / R), stamps).
+template <typename F, int N>
+__global__ void __launch_bounds__((Rows<F, N>::T), (Rows<F, N>::WAVES))
+row_pixels(gsmi_stamp* __restrict__ stamps, const cplx<F>* __restrict__ scratch,
+           TwiddleSet<F> tws, F* __restrict__ out)
+{
+    row_pixels_body<F, N, Rows<F, N>::T>(stamps + blockIdx.y, blockIdx.x, scratch, tws, out);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Several FFT sizes in one launch of each kernel, for batches of few stamps: a launch of a handful
+// of workgroups takes 6 to 12 us whatever its size, one per FFT size and kernel.  The bodies run
+// with kAnyT threads and the LDS of the largest size present, so a batch that fills the chip keeps
+// its launches per size, with the occupancy of each.
+// ---------------------------------------------------------------------------------------------
+constexpr int kAnyT = 512;
+constexpr int kMaxSizes = 16;
+struct SizeList {
+    int n;
+    int N[kMaxSizes];
+    int first[kMaxSizes];          // first stamp
+    int per[kMaxSizes];            // workgroups per stamp
+    int start[kMaxSizes + 1];      // first workgroup
+
+    __device__ __forceinline__ int find(int b, int* stamp, int* block) const
+    {
+        int k = 0;
+        while (k + 1 < n && b >= start[k + 1]) ++k;
+        const int r = b - start[k];
+        *stamp = first[k] + r / per[k];
+        *block = r % per[k];
+        return N[k];
+    }
+};
+
+#define GSMI_F32_SIZES(X) X(256) X(384) X(512) X(768) X(1024) X(1536) X(2048) X(3072) X(4096)
+#define GSMI_F64_SIZES(X) X(128) X(192) X(256) X(384) X(512) X(768) X(1024) X(1536) X(2048)
+
+template <typename F, int SIG>
+__global__ void __launch_bounds__(kAnyT, 2)
+fold_cols_any(gsmi_stamp* __restrict__ stamps, SizeList sizes, const gsmi_op* __restrict__ ops,
+              const gsmi_leaf* __restrict__ leaves, Tables<F> tb, TwiddleSet<F> tws, int lds_bytes,
+              cplx<F>* __restrict__ scratch)
+{
+    int stamp, block;
+    const int N = sizes.find(blockIdx.x, &stamp, &block);
+    switch (N) {
+#define GSMI_SIZE(NN)                                                                           \
+      case NN:                                                                                  \
+        fold_cols_body<F, NN, SIG, kAnyT>(stamps + stamp, block, ops, leaves, tb, tws,          \
+                                          lds_bytes, 1, scratch);                               \
+        break;
+#ifdef GSMI_WIDE_F64
+      GSMI_F64_SIZES(GSMI_SIZE)
+#else
+      GSMI_F32_SIZES(GSMI_SIZE)
+#endif
+#undef GSMI_SIZE
+    }
+}
+
+template <typename F>
+__global__ void __launch_bounds__(kAnyT, 2)
+row_pixels_any(gsmi_stamp* __restrict__ stamps, SizeList sizes,
+               const cplx<F>* __restrict__ scratch, TwiddleSet<F> tws, F* __restrict__ out)
+{
+    int stamp, block;
+    const int N = sizes.find(blockIdx.x, &stamp, &block);
+    switch (N) {
+#define GSMI_SIZE(NN)                                                                           \
+      case NN: row_pixels_body<F, NN, kAnyT>(stamps + stamp, block, scratch, tws, out); break;
+#ifdef GSMI_WIDE_F64
+      GSMI_F64_SIZES(GSMI_SIZE)
+#else
+      GSMI_F32_SIZES(GSMI_SIZE)
+#endif
+#undef GSMI_SIZE
+    }
+}
+
 template <typename F, int N, int SIG>
 int launch_cols(const gsmi_stamp* stamps, int nstamps, int ncoef, const gsmi_op* ops,
                 const gsmi_leaf* leaves, Tables<F> tb, TwiddleSet<F> tws,
@@ -411,6 +499,108 @@ int launch_wide_all(const gsmi_stamp* stamps, int nstamps, int max_ny, int ncoef
     for (int s0 = 0; s0 < nstamps && !rc; s0 += 32768)
         rc = launch_wide<F, N>(stamps + s0, nstamps - s0 < 32768 ? nstamps - s0 : 32768, max_ny,
                                ncoef, program, ops, leaves, tb, tws, scratch, out, stream);
+    return rc;
+}
+
+template <typename F>
+int launch_any(const gsmi_stamp* stamps, const SizeList& cols, const SizeList& rows, size_t lds_c,
+               size_t lds_r, int program, const gsmi_op* ops, const gsmi_leaf* leaves,
+               Tables<F> tb, TwiddleSet<F> tws, cplx<F>* scratch, F* out, void* stream)
+{
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    gsmi_stamp* st = const_cast<gsmi_stamp*>(stamps);
+    int rc = GSMI_E_ARG;
+    auto cols_of = [&](auto fn) {
+        rc = allow_lds(reinterpret_cast<const void*>(fn), lds_c);
+        if (rc) return;
+        hipLaunchKernelGGL(fn, dim3(cols.start[cols.n]), dim3(kAnyT), lds_c, s, st, cols, ops,
+                           leaves, tb, tws, int(lds_c), scratch);
+        rc = hip_check(hipGetLastError(), "fold_cols launch");
+    };
+    switch (program) {
+      case 1: cols_of(fold_cols_any<F, 1>); break;
+      case 2: cols_of(fold_cols_any<F, 2>); break;
+      case 3: cols_of(fold_cols_any<F, 3>); break;
+      case 4: cols_of(fold_cols_any<F, 4>); break;
+#ifndef GSMI_WIDE_F64
+      case kMoffatTableProgram: cols_of(fold_cols_any<F, kMoffatTableProgram>); break;
+#endif
+      default: set_error("unknown program shape");
+    }
+    if (rc) return rc;
+    auto fn = row_pixels_any<F>;
+    if ((rc = allow_lds(reinterpret_cast<const void*>(fn), lds_r))) return rc;
+    hipLaunchKernelGGL(fn, dim3(rows.start[rows.n]), dim3(kAnyT), lds_r, s, st, rows, scratch, tws,
+                       out);
+    return hip_check(hipGetLastError(), "row_pixels launch");
+}
+
+// Every group: one axis-factor launch over their stamps, then both kernels for all of them when
+// there are several sizes and few workgroups (below 1024 columns workgroups: 4 per CU, where
+// occupancy decides nothing yet), else size by size.
+template <typename F>
+int draw_groups(const gsmi_stamp* stamps, const gsmi_size_group* groups, int ngroups, int ncoef,
+                int program, const gsmi_op* ops, const gsmi_leaf* leaves, Tables<F> tb,
+                TwiddleSet<F> tws, cplx<F>* scratch, F* out, void* stream)
+{
+    SizeList cols{}, rows{};
+    size_t lds_c = 0, lds_r = 0;
+    int lo = 0x7fffffff, hi = 0;
+    int64_t blocks = 0;
+    for (int g = 0; g < ngroups; ++g) {
+        const gsmi_size_group& G = groups[g];
+        lo = G.first < lo ? G.first : lo;
+        hi = G.first + G.count > hi ? G.first + G.count : hi;
+        int chunks = 0, R = 1;
+        size_t c = 0, r = 0;
+        switch (G.N) {
+#define GSMI_SIZE(NN)                                                                           \
+          case NN:                                                                              \
+            chunks = NN / 2 / Cols<F, NN>::CC;                                                  \
+            R = Rows<F, NN>::R;                                                                 \
+            c = cols_lds<F, NN>(ncoef);                                                         \
+            r = rows_lds<F, NN>;                                                                \
+            break;
+#ifdef GSMI_WIDE_F64
+          GSMI_F64_SIZES(GSMI_SIZE)
+#else
+          GSMI_F32_SIZES(GSMI_SIZE)
+#endif
+#undef GSMI_SIZE
+        }
+        blocks += int64_t(G.count) * chunks;
+        if (blocks > 1024 || g >= kMaxSizes) continue;
+        lds_c = c > lds_c ? c : lds_c;
+        lds_r = r > lds_r ? r : lds_r;
+        cols.N[g] = rows.N[g] = G.N;
+        cols.first[g] = rows.first[g] = G.first;
+        cols.per[g] = chunks;
+        rows.per[g] = (G.max_ny + R - 1) / R;
+        cols.start[g + 1] = cols.start[g] + G.count * chunks;
+        rows.start[g + 1] = rows.start[g] + G.count * rows.per[g];
+        cols.n = rows.n = g + 1;
+    }
+    int rc = launch_axis_factors<F>(stamps + lo, hi - lo, ops, leaves, scratch, stream);
+    if (rc) return rc;
+    if (ngroups > 1 && ngroups <= kMaxSizes && blocks <= 1024)
+        return launch_any<F>(stamps, cols, rows, lds_c, lds_r, program, ops, leaves, tb, tws,
+                             scratch, out, stream);
+    for (int g = 0; g < ngroups && !rc; ++g) {
+        const gsmi_size_group& G = groups[g];
+        switch (G.N) {
+#define GSMI_SIZE(NN)                                                                           \
+          case NN:                                                                              \
+            rc = launch_wide_all<F, NN>(stamps + G.first, G.count, G.max_ny, ncoef, program,    \
+                                        ops, leaves, tb, tws, scratch, out, stream);            \
+            break;
+#ifdef GSMI_WIDE_F64
+          GSMI_F64_SIZES(GSMI_SIZE)
+#else
+          GSMI_F32_SIZES(GSMI_SIZE)
+#endif
+#undef GSMI_SIZE
+        }
+    }
     return rc;
 }
 

@@ -5,6 +5,7 @@ the profile tree into the k-space program of include/gsmi.h, packs the stamp rec
 leaves, Sersic tables and Exponential clip rows into one host buffer, copies it to the device
 in one transfer, and runs the two kernels of gsmi_draw_fft_f64/f32 on torch's current stream.
 """
+import ctypes
 import math
 import warnings
 
@@ -455,8 +456,9 @@ def draw_fft(prof, bounds, precision='f64', return_device=False, dest=None):
     program = _static_program(ctx, nops) if precision == 'f64' else 0
     if program and lib.gsmi_draw_wide_lds_f64(N, Nk) > 0:
         # (the specialised kernels' tiles are below any gfx950 limit: 107 KB of LDS at most)
-        rc = lib.gsmi_draw_wide_f64(base + o_stamp, 1, N, Nk, ny, program, base + o_ops,
-                                    base + o_leaves, base + o_tab, base + o_clip,
+        group = _lib.SizeGroup(N, 0, 1, ny, Nk)
+        rc = lib.gsmi_draw_wide_f64(base + o_stamp, ctypes.addressof(group), 1, program,
+                                    base + o_ops, base + o_leaves, base + o_tab, base + o_clip,
                                     scratch.data_ptr(), out.data_ptr(), stream)
     elif precision == 'f64':
         rc = lib.gsmi_draw_fft_f64(base + o_stamp, 1, N, ny, base + o_ops, base + o_leaves,

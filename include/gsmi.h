@@ -387,15 +387,22 @@ int gsmi_draw_stamps_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_N
                          const double* tables, const float* tables32, const void* scratch,
                          float* out, void* stream);
 /* The same for the larger sizes N = 2^k and 3 2^k from 256 to 4096, through the scratch buffer:
- * the axis-factor prepass, a kernel over packed columns and one over rows of at most max_ny,
- * compiled per size.  A stamp that breaks the conditions above has undefined pixels and
- * GSMI_STAMP_NONFINITE set. */
-int gsmi_draw_wide_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int max_ny,
+ * the axis-factor prepass, a kernel over packed columns and one over rows, compiled per size, for
+ * groups of stamps (in host memory).  A stamp that breaks the conditions above has undefined pixels
+ * and GSMI_STAMP_NONFINITE set.  The prepass runs over every stamp from the first group's first to
+ * the last one's last, clearing their status. */
+typedef struct gsmi_size_group {
+    int32_t N;            /* FFT size of the group's stamps                                   */
+    int32_t first, count; /* their range in the stamps array                                  */
+    int32_t max_ny;       /* at least the largest ny                                          */
+    int32_t max_Nk;       /* the largest Nk, N <= Nk < 2 N                                    */
+} gsmi_size_group;
+int gsmi_draw_wide_f32(const gsmi_stamp* stamps, const gsmi_size_group* groups, int ngroups,
                        int max_ncoef, int program, const gsmi_op* ops, const gsmi_leaf* leaves,
                        const double* tables, const float* tables32, void* scratch, float* out,
                        void* stream);
 /* The FP64 form, N = 2^k and 3 2^k from 128 to 2048, programs 1 to 4. */
-int gsmi_draw_wide_f64(const gsmi_stamp* stamps, int nstamps, int N, int max_Nk, int max_ny,
+int gsmi_draw_wide_f64(const gsmi_stamp* stamps, const gsmi_size_group* groups, int ngroups,
                        int program, const gsmi_op* ops, const gsmi_leaf* leaves,
                        const double* tables, const int32_t* cliprows, void* scratch, double* out,
                        void* stream);

@@ -177,3 +177,43 @@ def test_wide_fp64_matches_general_kernels(gal, psf, N):
         b = ref.stamp(3).cpu().numpy()
         assert np.abs(one - b).max() < 2e-14 * np.abs(b).max()
         assert not plan.status().any()
+
+
+@pytest.mark.parametrize("precision", ['f32', 'f64'])
+def test_sizes_drawn_together_and_apart(precision):
+    """Every wide size in one launch (few stamps) against each by itself, and beside a size the list
+    kernels draw (N = 64): their prepass leaves the other stamps' status alone."""
+    sizes = [64, 128, 192, 256, 384, 512, 768, 1024, 1536, 2048] + \
+        ([3072, 4096] if precision == 'f32' else [])
+    gsp = g.GSParams(minimum_fft_size=64)
+    profs, nx, ny = [], [], []
+    for i, N in enumerate(sizes):
+        e = g.Exponential(half_light_radius=0.1, flux=200., gsparams=gsp).shear(g1=0.2, g2=0.1)
+        profs.append(g.Convolve([e, g.Kolmogorov(fwhm=0.3, gsparams=gsp)]))
+        nx.append(N - i % 2)
+        ny.append(N if i % 3 else 19)
+    bad = {'f32': 1e38, 'f64': 1e306}[precision]
+    e = g.Exponential(half_light_radius=0.1, flux=bad, gsparams=gsp).shear(g1=0.2, g2=0.1)
+    profs += [g.Convolve([e, g.Kolmogorov(fwhm=0.3, flux=1e5, gsparams=gsp)])] * 2
+    nx, ny = np.array(nx + [128, 384]), np.array(ny + [100, 300])
+    plan = BatchPlan(profs, nx, ny, 0.1, precision=precision)
+    assert [x[0] for x in plan.list_groups] == [64]
+    for use in (False, True):
+        if use:
+            plan.use_schedule()
+        plan.out.fill_(7.)
+        plan.run()
+        st = plan.status()
+        assert (st[:-2] == 0).all() and (st[-2:] == _lib.STAMP_NONFINITE).all(), (use, st)
+        together = plan.out.clone()
+        for i in range(len(sizes)):
+            one = BatchPlan([profs[i]], nx[i], ny[i], 0.1, precision=precision)
+            one.run()
+            # the same bodies with another number of threads
+            assert _peak_rel(plan.stamp(i), one.stamp(0)) < (2e-7 if precision == 'f32' else 1e-15)
+    ref = _general(BatchPlan(profs[:-2], nx[:-2], ny[:-2], 0.1, precision='f64')) \
+        if precision == 'f64' else None
+    if ref is not None:
+        for i in range(len(sizes)):
+            a = together[int(plan.stamp_offset[i]):][:int(nx[i] * ny[i])]
+            assert _peak_rel(a, ref.stamp(i).reshape(-1)) < 2e-14
