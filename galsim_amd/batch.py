@@ -150,6 +150,11 @@ def _program_shape(recs, ops, leaves):
 
 
 FOLD_ITEM_CELLS = 16384       # default size of a fold work item (columns x N), in cells
+# A workgroup takes 20 us (N = 128) to 37 us (192) over a whole bulge + disk stamp, however few
+# there are: below this many the column and row kernels, which spread a stamp over the CUs, are
+# faster (bulge + disk batches of 32, 128 and 192 stamps, us: 82, 87, 97 by one workgroup per
+# stamp, 24, 53, 120 by columns and rows; Exponential x Kolmogorov ones 43, 43, 43 and 21, 38, 49)
+STAMP_MIN = 128
 LIST_LDS_LIMIT = 163840       # LDS one workgroup may allocate on gfx950 (160 KiB)
 
 
@@ -384,18 +389,21 @@ class BatchPlan:
         self._rerun_cleared = np.zeros(n, dtype=bool)
         self.nops = len(host_ops)
         self.nleaves = len(host_leaves)
-        self.stamp_groups, self.wide_groups, self.list_groups = self._split_groups()
+        self.stamp_fit, self.wide_groups, self.list_groups = self._split_groups()
+        self.stamp_groups = self.stamp_fit
+        if sum(g[2] for g in self.stamp_fit) < STAMP_MIN:
+            self.stamp_groups, self.wide_groups = [], self.stamp_fit + self.wide_groups
         self._sched = None
         self._graph = None
         self.tuning = None
 
     def _split_groups(self):
-        """(stamp groups, wide groups, list groups): how each FFT size is drawn.  Batches of a
+        """(stamp groups, wide groups, list groups): how each FFT size can be drawn.  Batches of a
         specialised program shape whose stamps have Nk < 2 N (at most one alias per axis, which is
         what the cell passes of these kernels add) take the kernels compiled per size: in FP32 one
         workgroup per stamp at N = 128 and 192, whose wrapped grid fits its LDS
-        (gsmi_draw_stamps_f32), and a column and a row kernel from 256 to 4096
-        (gsmi_draw_wide_f32); in FP64 those two from 128 to 2048 (gsmi_draw_wide_f64); each
+        (gsmi_draw_stamps_f32; STAMP_MIN decides), and a column and a row kernel from 128 to
+        4096 (gsmi_draw_wide_f32); in FP64 those two from 128 to 2048 (gsmi_draw_wide_f64); each
         (N, first, count, max_ny, largest Nk, Sersic coefficients).  Everything else, as
         (N, first, count, max_ny), takes the fold and row kernels of any shape and size."""
         if not self.program_shape:

@@ -1,5 +1,5 @@
 // Drawing of stamps of a specialised program shape in two kernels compiled per FFT size (FP32 at
-// N = 256 to 4096, FP64 at 128 to 2048): columns of the wrapped grid to the scratch buffer, then
+// N = 128 to 4096, FP64 at 128 to 2048): columns of the wrapped grid to the scratch buffer, then
 // its rows to pixels.
 //
 // fold_cols: a workgroup takes CC packed columns at a time: fill_cells puts their cells in LDS, an
@@ -90,6 +90,8 @@ struct Cols;
         static constexpr bool lds_tw = N <= 2048;                                               \
         static_assert(CC % 2 == 0 && (N / 2) % CC == 0, "even chunks that divide the columns");  \
     };
+GSMI_COLS(float, 128, 8, 16, 1, 16, 256, 4)
+GSMI_COLS(float, 192, 12, 16, 1, 12, 256, 4)
 GSMI_COLS(float, 256, 16, 16, 1, 16, 256, 4)
 GSMI_COLS(float, 384, 12, 4, 8, 8, 256, 4)
 GSMI_COLS(float, 512, 8, 8, 8, 8, 256, 3)
@@ -118,6 +120,8 @@ struct Rows;
     struct Rows<F, N> : Line<N / 2, D1, D2, D3> {                                               \
         static constexpr int R = R_, T = T_, WAVES = WAVES_;                                    \
     };
+GSMI_ROWS(float, 128, 8, 8, 1, 32, 128, 4)
+GSMI_ROWS(float, 192, 8, 12, 1, 32, 256, 4)
 GSMI_ROWS(float, 256, 8, 16, 1, 32, 256, 4)
 GSMI_ROWS(float, 384, 12, 16, 1, 32, 256, 3)
 GSMI_ROWS(float, 512, 8, 8, 4, 16, 256, 4)
@@ -361,11 +365,17 @@ row_pixels(gsmi_stamp* __restrict__ stamps, const cplx<F>* __restrict__ scratch,
 }
 
 // ---------------------------------------------------------------------------------------------
-// Several FFT sizes in one launch of each kernel, for batches of few stamps: a launch of a handful
-// of workgroups takes 6 to 12 us whatever its size, one per FFT size and kernel.  The bodies run
-// with kAnyT threads and the LDS of the largest size present, so a batch that fills the chip keeps
-// its launches per size, with the occupancy of each.
+// Several FFT sizes in one launch of each kernel: a launch of a handful of workgroups takes 6 to
+// 12 us whatever its size, one per FFT size and kernel, and each launch has a tail.  The bodies run
+// with kAnyT threads and the LDS of the largest size present, so beyond kMergeBlocks column
+// workgroups (64 per CU) the launches per size win by their occupancy.  Measured, apart |
+// together, us: bulge + disk batches of 400 stamps (1080 workgroups) 180 | 127, 2400 (4696) 423 |
+// 387, 4096 (8968) 636 | 625; Sersic batches of 16 (5248) 385 | 312, 48 (13752) 823 | 787, 64
+// (24064) 1283 | 1330.  FP64, whose bodies hold 512-thread workgroups to two waves per SIMD, ends
+// at 4 per CU: 256 stamps of two sizes (2300) 80 | 130.
 // ---------------------------------------------------------------------------------------------
+template <typename F>
+constexpr int kMergeBlocks = sizeof(F) == 4 ? 16384 : 1024;
 constexpr int kAnyT = 512;
 constexpr int kMaxSizes = 16;
 struct SizeList {
@@ -386,11 +396,12 @@ struct SizeList {
     }
 };
 
-#define GSMI_F32_SIZES(X) X(256) X(384) X(512) X(768) X(1024) X(1536) X(2048) X(3072) X(4096)
+#define GSMI_F32_SIZES(X) X(128) X(192) X(256) X(384) X(512) X(768) X(1024) X(1536) X(2048) \
+    X(3072) X(4096)
 #define GSMI_F64_SIZES(X) X(128) X(192) X(256) X(384) X(512) X(768) X(1024) X(1536) X(2048)
 
 template <typename F, int SIG>
-__global__ void __launch_bounds__(kAnyT, 2)
+__global__ void __launch_bounds__(kAnyT, (sizeof(F) == 4 ? 4 : 2))
 fold_cols_any(gsmi_stamp* __restrict__ stamps, SizeList sizes, const gsmi_op* __restrict__ ops,
               const gsmi_leaf* __restrict__ leaves, Tables<F> tb, TwiddleSet<F> tws, int lds_bytes,
               cplx<F>* __restrict__ scratch)
@@ -413,7 +424,7 @@ fold_cols_any(gsmi_stamp* __restrict__ stamps, SizeList sizes, const gsmi_op* __
 }
 
 template <typename F>
-__global__ void __launch_bounds__(kAnyT, 2)
+__global__ void __launch_bounds__(kAnyT, (sizeof(F) == 4 ? 4 : 2))
 row_pixels_any(gsmi_stamp* __restrict__ stamps, SizeList sizes,
                const cplx<F>* __restrict__ scratch, TwiddleSet<F> tws, F* __restrict__ out)
 {
@@ -536,8 +547,7 @@ int launch_any(const gsmi_stamp* stamps, const SizeList& cols, const SizeList& r
 }
 
 // Every group: one axis-factor launch over their stamps, then both kernels for all of them when
-// there are several sizes and few workgroups (below 1024 columns workgroups: 4 per CU, where
-// occupancy decides nothing yet), else size by size.
+// there are several sizes and at most kMergeBlocks column workgroups, else size by size.
 template <typename F>
 int draw_groups(const gsmi_stamp* stamps, const gsmi_size_group* groups, int ngroups, int ncoef,
                 int program, const gsmi_op* ops, const gsmi_leaf* leaves, Tables<F> tb,
@@ -569,7 +579,7 @@ int draw_groups(const gsmi_stamp* stamps, const gsmi_size_group* groups, int ngr
 #undef GSMI_SIZE
         }
         blocks += int64_t(G.count) * chunks;
-        if (blocks > 1024 || g >= kMaxSizes) continue;
+        if (blocks > kMergeBlocks<F> || g >= kMaxSizes) continue;
         lds_c = c > lds_c ? c : lds_c;
         lds_r = r > lds_r ? r : lds_r;
         cols.N[g] = rows.N[g] = G.N;
@@ -582,7 +592,7 @@ int draw_groups(const gsmi_stamp* stamps, const gsmi_size_group* groups, int ngr
     }
     int rc = launch_axis_factors<F>(stamps + lo, hi - lo, ops, leaves, scratch, stream);
     if (rc) return rc;
-    if (ngroups > 1 && ngroups <= kMaxSizes && blocks <= 1024)
+    if (ngroups > 1 && ngroups <= kMaxSizes && blocks <= kMergeBlocks<F>)
         return launch_any<F>(stamps, cols, rows, lds_c, lds_r, program, ops, leaves, tb, tws,
                              scratch, out, stream);
     for (int g = 0; g < ngroups && !rc; ++g) {

@@ -107,9 +107,8 @@ class DiffPlan:
         lib = _lib.lib()
         need = 1
         self._bins = []
-        # sizes the forward draws by one workgroup per stamp: their adjoint does the same
-        self._stamp_bins = [(N, first, count, nk) for N, first, count, _, nk, _ in
-                            p.stamp_groups]
+        # sizes whose grid one workgroup holds
+        self._stamp_bins = [(N, first, count, nk) for N, first, count, _, nk, _ in p.stamp_fit]
         whole = {b[0] for b in self._stamp_bins}
         for N, first, count, max_ny in p.groups:
             if N in whole:

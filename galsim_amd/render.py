@@ -386,9 +386,13 @@ def store(t, dest):
     n = flat.numel()
     total = flat.sum(dtype=torch.float64) if n >= DEVICE_SUM else None
     step = STAGE_BYTES // t.element_size()
+    if n <= step:
+        block = torch.empty(n, dtype=t.dtype, pin_memory=True)
+        block.copy_(flat)
+        out.copy_(block)
+        return float(block.numpy().sum(dtype=float)) if total is None else float(total)
     spans = [(a, min(a + step, n)) for a in range(0, n, step)]
-    blocks = [torch.empty(min(step, n), dtype=t.dtype, pin_memory=True)
-              for _ in range(min(2, len(spans)))]
+    blocks = [torch.empty(step, dtype=t.dtype, pin_memory=True) for _ in range(2)]
     ready = [torch.cuda.Event() for _ in blocks]
 
     def fetch(k):
@@ -403,9 +407,7 @@ def store(t, dest):
         out[a:b].copy_(blocks[k % 2][:b - a])
         if k + 2 < len(spans):
             fetch(k + 2)
-    if total is not None:
-        return float(total)
-    return float(blocks[0].numpy().sum(dtype=float)) if n else 0.
+    return float(total)
 
 
 def _device_buffer(torch, packer):

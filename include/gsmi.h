@@ -386,7 +386,7 @@ int gsmi_draw_stamps_f32(const gsmi_stamp* stamps, int nstamps, int N, int max_N
                          int program, const gsmi_op* ops, const gsmi_leaf* leaves,
                          const double* tables, const float* tables32, const void* scratch,
                          float* out, void* stream);
-/* The same for the larger sizes N = 2^k and 3 2^k from 256 to 4096, through the scratch buffer:
+/* The same for N = 2^k and 3 2^k from 128 to 4096, through the scratch buffer:
  * the axis-factor prepass, a kernel over packed columns and one over rows, compiled per size, for
  * groups of stamps (in host memory).  A stamp that breaks the conditions above has undefined pixels
  * and GSMI_STAMP_NONFINITE set.  The prepass runs over every stamp from the first group's first to

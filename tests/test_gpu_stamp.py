@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import galsim_amd as g
-from galsim_amd import _lib
+from galsim_amd import _lib, batch
 from galsim_amd.batch import BatchPlan
 
 pytestmark = pytest.mark.gpu
@@ -48,7 +48,9 @@ SHAPES = [('bulge_disk', 'kolmogorov'), ('exp', 'moffat3'), ('exp', 'moffat2.5')
 
 @pytest.mark.parametrize("gal,psf", SHAPES)
 @pytest.mark.parametrize("scale", [0.13, 0.2, 0.28])
-def test_stamps_match_fp64_and_list_kernels(gal, psf, scale):
+@pytest.mark.parametrize("whole", [True, False])
+def test_stamps_match_fp64_and_list_kernels(gal, psf, scale, whole, monkeypatch):
+    monkeypatch.setattr(batch, 'STAMP_MIN', 0 if whole else 1000)
     sides = [(1, 1), (2, 3), (64, 64), (63, 65), (127, 128), (128, 127), (128, 128), (129, 40),
              (190, 191), (192, 192), (33, 192)]
     rng = np.random.default_rng(int(100 * scale) + len(gal) + len(psf))
@@ -62,7 +64,8 @@ def test_stamps_match_fp64_and_list_kernels(gal, psf, scale):
         profs.append(g.Convolve([_gal(gal, hlr, gm * np.cos(2 * ph), gm * np.sin(2 * ph)), p]))
     nx, ny = np.array(sides).T
     plan = BatchPlan(profs, nx, ny, scale, offs, precision='f32')
-    assert {x[0] for x in plan.stamp_groups} <= {128, 192} and plan.stamp_groups
+    assert {x[0] for x in plan.stamp_fit} <= {128, 192} and plan.stamp_fit
+    assert bool(plan.stamp_groups) == whole
     plan.out.fill_(float('nan'))
     plan.run()
     lists = _general(BatchPlan(profs, nx, ny, scale, offs, precision='f32'))
@@ -73,8 +76,9 @@ def test_stamps_match_fp64_and_list_kernels(gal, psf, scale):
     assert not plan.status().any()
 
 
-def test_stamp_path_is_left_for_other_sizes_and_shapes():
+def test_stamp_path_is_left_for_other_sizes_and_shapes(monkeypatch):
     """Beyond one alias per axis, another program shape, or FP64: the fold and row kernels."""
+    monkeypatch.setattr(batch, 'STAMP_MIN', 0)
     def plan(prof, scale=0.2, precision='f32'):
         return BatchPlan([prof] * 2, 64, 64, scale, precision=precision)
     e, m = g.Exponential(half_light_radius=0.4), g.Moffat(beta=3, fwhm=0.7)
@@ -93,10 +97,11 @@ def test_stamp_path_is_left_for_other_sizes_and_shapes():
     assert _peak_rel(coarse.stamp(0), ref.stamp(0)) < TOL
 
 
-def test_stamp_status_and_rejected_stamps():
+def test_stamp_status_and_rejected_stamps(monkeypatch):
     """A stamp whose flux overflows FP32 is flagged and the next run clears the flag; a record
     that is not of the launch's size is left undrawn and flagged."""
     import torch
+    monkeypatch.setattr(batch, 'STAMP_MIN', 0)
     e, m = g.Exponential(half_light_radius=0.6, flux=1e3), g.Moffat(beta=3, fwhm=0.7)
     profs = [g.Convolve([e, m]), g.Convolve([e.withFlux(1e38), m.withFlux(1e5)]),
              g.Convolve([e, m])]
