@@ -678,41 +678,38 @@ def main():
     recs = plan.recs
     nfac = {}
     flops = {'fold': 0., 'rows': 0.}
-    nbytes = {'fold': 0., 'rows': 0.}
     for r in recs:
         rec = (int(r['N']), int(r['Nk']), int(r['ny']), r['op_count'])
         # factors: LEAF + PHASE + SCALE ops (each a complex multiply-accumulate per sample)
         f, rw = kernel_flops((rec[0], rec[1], rec[2], 5))
         flops['fold'] += f
         flops['rows'] += rw
-        bf, br = kernel_bytes((rec[0], rec[1], rec[2], 5), int(r['nx']), 4)
-        nbytes['fold'] += bf
-        nbytes['rows'] += br
+    # the whole step: the kernels compiled per FFT size (one workgroup per stamp at N = 128 and
+    # 192, which touches memory for its pixels only; columns and rows above), and the fold and
+    # row work lists of any size they do not take
     t_fold = sum(fold_ms.values())
     t_rows = sum(rows_ms.values())
-    n_launch = len(fold_ms)
-    dominant = 'fold' if t_fold >= t_rows else 'rows'
-    t_dom = t_fold if dominant == 'fold' else t_rows
-    achieved = flops[dominant] / (t_dom * 1e-3) / 1e12
-    log("work lists: fold %.3f ms/step over %d launch(es); rows %.3f ms/step" % (
-        t_fold, n_launch, t_rows))
-    traffic = None
-    tfile = os.path.join(ROOT, 'profiles', 'hbm_traffic_bulge_disk_4096.json')
-    if os.path.exists(tfile):
-        with open(tfile) as f:
-            traffic = json.load(f).get(dominant + '_list')
+    t_dom = t_fold + t_rows
+    in_lds = {g[0] for g in plan.stamp_groups}
+    step_bytes = sum(4. * int(r['nx']) * int(r['ny']) if int(r['N']) in in_lds else
+                     sum(kernel_bytes((int(r['N']), int(r['Nk']), int(r['ny']), 5), int(r['nx']),
+                                      4)) for r in recs)
+    n_launch = len(plan.stamp_groups) + (3 if plan.wide_groups else 0) + \
+        (3 if plan.list_groups else 0)
+    achieved = (flops['fold'] + flops['rows']) / (t_dom * 1e-3) / 1e12
+    log("step: %.3f ms of kernels over %d launches" % (t_dom, n_launch))
     roofline = {
-        "kernel": "fold_list_f32" if dominant == 'fold' else "rows_list<float>",
-        # vector ALU issue bounds the kernel (no matrix-core work on this path)
+        "kernel": "draw_stamp_f32 + fold_cols + row_pixels (the whole step)",
+        # vector ALU issue bounds the kernels (no matrix-core work on this path)
         "bound": "valu",
         "achieved": round(achieved, 4),
         "peak": FP32_PEAK_TFLOPS,
         "unit": "TFLOP/s",
         "frac": round(achieved / FP32_PEAK_TFLOPS, 6),
-        "traffic": traffic,
-        "algorithmic_bytes_per_step": nbytes[dominant],
-        "hbm_GBps_algorithmic": round(nbytes[dominant] / (t_dom * 1e-3) / 1e9, 2),
-        "hbm_frac_algorithmic": round(nbytes[dominant] / (t_dom * 1e-3) / 1e9 / HBM_PEAK_GBS, 6),
+        "traffic": None,
+        "algorithmic_bytes_per_step": step_bytes,
+        "hbm_GBps_algorithmic": round(step_bytes / (t_dom * 1e-3) / 1e9, 2),
+        "hbm_frac_algorithmic": round(step_bytes / (t_dom * 1e-3) / 1e9 / HBM_PEAK_GBS, 6),
         "avg_launch_ms": round(t_dom / max(n_launch, 1), 5),
         "launches_per_step": n_launch,
         "frac_of_nonpacked_fp32_peak": round(achieved / FP32_NONPACKED_TFLOPS, 6),
@@ -867,7 +864,8 @@ def main():
         "end_to_end_config_stamps_per_s": round(e2e_rate, 1),
         "end_to_end_note": "config-driven planning (vectorised) + one host-to-device copy of "
                            "the records + the tuned launches, output left on the device",
-        "schedule": {"launches": "axis prepass + 1 fold + 1 row launch per step, replayed "
+        "schedule": {"launches": "one launch per FFT size that a workgroup holds, an axis "
+                                 "prepass, a column and a row launch for the others, replayed "
                                  "from one HIP graph",
                      "cols_per_group": {str(k): v for k, v in tuning['cols'].items()},
                      "rows_per_group": {str(k): v for k, v in tuning['rows'].items()},
