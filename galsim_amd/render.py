@@ -360,6 +360,7 @@ class _Packer:
         return buf
 
 
+THREADED_SUM = 65536           # pixels from which torch's threads take the sum: _host_sum
 STAGE_BYTES = 4 << 20          # one of the two pinned blocks a device-to-host copy goes through
 
 
@@ -371,6 +372,18 @@ def direct_array(image, add_to_image):
     return a if ok else None
 
 
+def _host_sum(block):
+    """The sum of a host tensor's values in double: torch's threads from THREADED_SUM pixels.
+
+    Alone, numpy and torch took 8.5 and 6.6 us at 65536 FP64 pixels, 60 and 10 us at 524288, and
+    1.8 and 1.6 us at 4096; but a whole 64 x 64 drawImage call took 171 us with numpy's sum and
+    178 us with torch's."""
+    if block.numel() < THREADED_SUM:
+        return float(block.numpy().sum(dtype=float))
+    import torch
+    return float(block.sum(dtype=torch.float64))
+
+
 def store(t, dest):
     """Copy a contiguous device tensor into a C-contiguous float array of its shape, converting,
     and return the sum of the tensor's values in double.
@@ -378,11 +391,10 @@ def store(t, dest):
     The rows come through two pinned blocks of at most STAGE_BYTES, one filled by the device while
     the other is written out.  A copy to pageable memory is staged by the runtime anyway, into an
     array that is then converted and copied twice more: a 1024 x 1000 FP64 image took 0.93 ms that
-    way and 0.23 ms this way.  The sum is torch's over the pinned blocks:
-    1.6 us at 4096 FP64 pixels, 6.6 us at 65536 and 10 us at 524288, where numpy's took 1.8, 8.5
-    and 60 us.  A device reduction was no faster for a whole drawImage call (565 us against 560 us
-    at 1001 x 769, 570 us against 544 us at 1000 x 1024), and 64 first draws in a process, 64 to
-    256 pixels wide, took 87 ms with it from 65536 pixels up and 49 ms without."""
+    way and 0.23 ms this way.  The sum is taken from the pinned blocks.
+    A device reduction was no faster for a whole drawImage call (565 us against 560 us at 1001 x
+    769, 570 us against 544 us at 1000 x 1024), and 64 first draws in a process, 64 to 256 pixels
+    wide, took 87 ms with it from 65536 pixels up and 49 ms without."""
     import torch
     flat, out = t.reshape(-1), torch.from_numpy(dest.reshape(-1))
     n = flat.numel()
@@ -391,7 +403,7 @@ def store(t, dest):
         block = torch.empty(n, dtype=t.dtype, pin_memory=True)
         block.copy_(flat)
         out.copy_(block)
-        return float(block.sum(dtype=torch.float64))
+        return _host_sum(block)
     spans = [(a, min(a + step, n)) for a in range(0, n, step)]
     blocks = [torch.empty(step, dtype=t.dtype, pin_memory=True) for _ in range(2)]
     ready = [torch.cuda.Event() for _ in blocks]
@@ -407,7 +419,7 @@ def store(t, dest):
     for k, (a, b) in enumerate(spans):
         ready[k % 2].synchronize()
         out[a:b].copy_(blocks[k % 2][:b - a])
-        total += float(blocks[k % 2][:b - a].sum(dtype=torch.float64))
+        total += _host_sum(blocks[k % 2][:b - a])
         if k + 2 < len(spans):
             fetch(k + 2)
     return total
